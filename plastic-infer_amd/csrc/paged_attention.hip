@@ -283,12 +283,16 @@ using PoolIn = std::conditional_t<APPEND, const uint16_t*, const uint16_t* __res
 // The wave keeps up to SD_APP_REC pending slots in LDS and stores any further ones at once.
 // The stores are non-temporal (streamed through the cache): the next step reads these lines
 // from another XCD, and that read was measured 0.4 % faster than after ordinary stores.
-// A wave's arrival on the counter of a cut segment with n partials: the counter holds
+// Arrivals of the n waves that hold partials of a cut segment: the segment's counter holds
 // (token << 16 | count) where token identifies the launch (the upper 48 bits, from the host, a
-// fresh value per launch); a count under another token is stale (an earlier launch, or a
-// workspace never used before) and reads as 0. Returns true for the n-th arrival, which also
-// leaves the count at 0 under this token, so a replay of the same launch (a graph) starts from
-// zero again. Workspace contents collide with a token with probability 2^-48.
+// fresh value per launch). Every wave of the segment first makes sure that the counter carries
+// the token (sd_install, at the start of its range, under its first loads: a count under
+// another token is stale, from an earlier launch or a workspace never used before), then counts
+// itself in with one atomic add after its range. The n-th arrival merges; it also leaves the
+// count at 0 under this token, so a replay of the same launch (a graph) starts from zero again.
+// Workspace contents collide with a token with probability 2^-48. (Counting in with a
+// compare-and-swap loop instead costs a round trip per lost race: one sequence of 3001 tokens,
+// 24 pieces per head that end together, took 24.4 us with the loop and 17.8 us with this.)
 // Device-coherent partial stores and loads (sc1: through the XCD's L2 to memory).
 __device__ __forceinline__ void sd_store(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -298,17 +302,24 @@ __device__ __forceinline__ float sd_load(const float* p) {
 }
 
 __device__ __forceinline__ bool sd_arrive(uint64_t* ctr, uint64_t token, int n) {
-  uint64_t old = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  for (;;) {  // retried only when another wave updated the counter in between
-    const uint64_t cnt = (old >> 16) == (token >> 16) ? (old & 0xffffu) : 0u;
-    const bool last = int(cnt) + 1 >= n;
-    const uint64_t nv = token | (last ? 0u : cnt + 1);
-    uint64_t expect = old;
-    if (__hip_atomic_compare_exchange_strong(ctr, &expect, nv, __ATOMIC_RELAXED,
-                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      return last;
-    old = expect;
-  }
+  const uint64_t prev = __hip_atomic_fetch_add(ctr, uint64_t(1), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+  if (int(prev & 0xffffu) + 1 < n) return false;
+  __hip_atomic_store(ctr, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// The launch's token onto a counter last seen holding `old`, before any arrival of this wave:
+// only waves of this launch touch the counter, so where the exchange fails another of them has
+// installed the token (and perhaps counted itself in).
+__device__ __forceinline__ void sd_install(uint64_t* ctr, uint64_t old, uint64_t token) {
+  if ((old >> 16) != (token >> 16))
+    __hip_atomic_compare_exchange_strong(ctr, &old, token, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ uint64_t* sd_counters(int32_t* ws_meta) {
+  return reinterpret_cast<uint64_t*>((reinterpret_cast<uintptr_t>(ws_meta) + 7) & ~uintptr_t(7));
 }
 
 // Step prefix of the batch, built by every wave in its own LDS copy: seq_q[b] = steps of the
@@ -442,8 +453,7 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
                                                     int lane) {
   constexpr int D = FD_D;
   if (arr_first[0] < 0 && arr_first[1] < 0) return;
-  uint64_t* ctr = reinterpret_cast<uint64_t*>(
-      (reinterpret_cast<uintptr_t>(ws_meta) + 7) & ~uintptr_t(7));
+  uint64_t* ctr = sd_counters(ws_meta);
   const int inc = Ce < Dp ? 1 : 2;  // odd waves hold no steps when pairs have one step
   __builtin_amdgcn_s_waitcnt(0);  // this wave's partial stores have completed before its count
   bool merge[2] = {false, false};
@@ -470,8 +480,8 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
       M[g] = kNegBig;
       o0[g] = o1[g] = lt[g] = 0.f;
     }
-    // pieces four at a time: all their loads in flight together, then folded in order
-    constexpr int PB = 4;
+    // pieces eight (G <= 4) or four at a time: their loads in flight together, folded in order
+    constexpr int PB = G <= 4 ? 8 : 4;
     for (int cb = c0; cb <= c1; cb += PB * inc) {
       float mc[PB][G], lc[PB][G], a0[PB][G], a1[PB][G];
 #pragma unroll
@@ -510,6 +520,31 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
     }
   }
 }
+
+// The counters of the (at most two) cut segments of a wave's range: read by begin() ahead of the
+// range's first loads, given the launch's token by finish() behind them.
+struct SegmentCounters {
+  uint64_t* ctr[2] = {nullptr, nullptr};
+  uint64_t old[2] = {0, 0};
+
+  __device__ __forceinline__ void begin(const StreamPlan& plan, const StreamCursor& first, int start,
+                                        int end, int Dp, int Ce, int32_t* ws_meta, int lane) {
+    uint64_t* base = sd_counters(ws_meta);
+    if (first.ls > 0) ctr[0] = base + stream_range_of(start - first.ls, Dp, Ce);
+    const StreamCursor last = plan.seg_of(end - 1);
+    const int f = end - 1 - last.ls;  // first step of the range's last segment
+    if (f >= start && f + last.ns > end) ctr[1] = base + stream_range_of(f, Dp, Ce);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (ctr[k] && lane == 0)
+        old[k] = __hip_atomic_load(ctr[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ void finish(uint64_t token, int lane) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      if (ctr[k] && lane == 0) sd_install(ctr[k], old[k], token);
+  }
+};
 
 template <int G, bool APPEND, int DT>
 __global__ __launch_bounds__(64, 2) void paged_decode_stream(
@@ -610,11 +645,14 @@ __global__ __launch_bounds__(64, 2) void paged_decode_stream(
     QRows q0;
     load_q(cur, q0);
     bt_cur = load_bt(cur);
+    SegmentCounters counters;
+    counters.begin(plan, cur, start, end, Dp, Ce, ws_meta, lane);
     const uint16_t* kp = kbase + int64_t(cur.h) * TILE + page_ok(bt_cur) * page_stride;
 #pragma unroll
     for (int i = 0; i < 16; ++i) bufA[i] = load16_nt(kp + 64 * i);
 #pragma unroll
     for (int i = 0; i < 16; ++i) bufB[i] = load16_nt(kp + 64 * (16 + i));
+    counters.finish(token, lane);
     stage_q(q0);
     __syncthreads();
   }
@@ -910,10 +948,11 @@ __global__ __launch_bounds__(64, 2) void paged_decode_stream(
     bt_cur = bt_nxt;
     ++gs;
   }
-  if constexpr (APPEND) sd_flush_appends(app_rec, n_rec, k_new, v_new, kpool_w, vpool_w, lane);
-  // All arrivals at the end of the range, so no fence drains a step's prefetch.
+  // All arrivals at the end of the range, so no fence drains a step's prefetch, and ahead of the
+  // new-token stores, which no other wave waits for.
   sd_arrive_and_merge<G, DT>(arr_first, arr_ns, arr_row, Dp, Ce, ws_part, ws_meta, token, out, Hkv,
                          lane);
+  if constexpr (APPEND) sd_flush_appends(app_rec, n_rec, k_new, v_new, kpool_w, vpool_w, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1162,9 +1201,12 @@ __global__ __launch_bounds__(64, 1) void paged_decode_mfma(
   int arr_first[2] = {-1, -1}, arr_ns[2] = {0, 0}, arr_row[2] = {0, 0};
   load_q(cur, qreg);
   int bt_cur = load_bt(cur);
+  SegmentCounters counters;
+  counters.begin(plan, cur, start, end, Dp, Ce, ws_meta, lane);
   uint4 bufA[16], bufB[16];
   load_k(bufA, cur.h, bt_cur, 0);
   load_k(bufB, cur.h, bt_cur, 1);
+  counters.finish(token, lane);
 
   for (;;) {
     {  // issue priority from progress: quartile 0 of the range -> 3, quartile 3 -> 0
@@ -1358,9 +1400,9 @@ __global__ __launch_bounds__(64, 1) void paged_decode_mfma(
     bt_cur = bt_nxt;
     ++gs;
   }
-  if constexpr (APPEND) sd_flush_appends(app_rec, n_rec, k_new, v_new, kpool_w, vpool_w, lane);
   sd_arrive_and_merge<G, DT>(arr_first, arr_ns, arr_row, Dp, Ce, ws_part, ws_meta, token, out, Hkv,
                          lane);
+  if constexpr (APPEND) sd_flush_appends(app_rec, n_rec, k_new, v_new, kpool_w, vpool_w, lane);
 }
 
 // ---------------------------------------------------------------------------------------------
