@@ -128,7 +128,8 @@ int pia_kv_pages_chunks_copy(void* const* chunks, int num_chunks, void* pages,
  * bf16 or fp16 with head_dim 128 and page_size 16 and Hq/Hkv in 1..8 or 16 takes the fast
  * kernel (the batch's KV steps split over persistent waves, XCD-aware; the probabilities enter
  * the P.V products rounded to the pools' dtype); every other supported combination
- * (f32/f16/bf16, head_dim <= 512, any page_size) takes the general kernel.
+ * (f32/f16/bf16, head_dim <= 512, any page_size) computes in fp32: over persistent waves when the
+ * workspace holds pia_paged_decode_split_scratch_bytes, else in the general kernel.
  * ------------------------------------------------------------------------------------------- */
 int64_t pia_paged_decode_workspace_bytes(int num_seqs, int num_heads, int num_kv_heads,
                                          int head_dim, int page_size, int64_t bt_stride);
@@ -143,6 +144,14 @@ int64_t pia_paged_decode_workspace_bytes(int num_seqs, int num_heads, int num_kv
  * PIA_EUNSUPPORTED (Hq / Hkv outside 1..8 and 16). */
 int pia_paged_decode_scratch_layout(int num_heads, int num_kv_heads, int waves,
                                     int64_t* partials_offset, int64_t* total_bytes);
+
+/* Scratch with which the other shapes run a kernel that, like the fast one, splits the batch over
+ * persistent waves (head_dim 64 or 128, Hq/Hkv up to 16, pages of whole 16-byte vectors; all
+ * products in fp32): passed as `workspace` to the two decode calls below, under the same ordering
+ * rule. It is optional: without it (NULL or fewer bytes) those shapes take the general kernel.
+ * 0: the shape has no such kernel. No counterpart in the reference. */
+int64_t pia_paged_decode_split_scratch_bytes(int num_heads, int num_kv_heads, int head_dim,
+                                             int page_size, int dtype);
 
 int pia_paged_decode_attention(void* out, const void* q, int64_t q_seq_stride,
                                const void* k_pages, const void* v_pages,

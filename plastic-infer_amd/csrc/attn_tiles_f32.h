@@ -1,24 +1,32 @@
-// Building blocks of the paged attention kernels that run on the fp32 matrix cores
-// (v_mfma_f32_16x16x4_f32, gfx950) for any storage type: 16-bit K / V elements are widened in
-// registers, probabilities and sums stay fp32.
-//
-// Operand layouts of v_mfma_f32_16x16x4_f32 (lane l, kd = l / 16, n16 = l % 16):
-//   A (16 x 4): lane l holds A[n16][kd]      B (4 x 16): lane l holds B[kd][n16]
-//   C (16 x 16): lane l holds C[4 kd + v][n16], v < 4
+// Building blocks of the paged attention kernels that keep full fp32 precision for any storage
+// type on the matrix cores of gfx950, with no LDS between memory and the MFMA operands.
 //
 // The pool's rows are [d][token], so a 16-byte vector of a row is TV = 4 (fp32) or 8 (16-bit)
-// consecutive tokens of one d, and K and V go from memory straight into MFMA operands, with no
-// LDS: a tile is 16 vectors (64 or 128 tokens), vector x = tokens TV x .. TV x + TV - 1.
-//   S^T = K . Q^T  lane l loads vector x = 4 (n16 % 4) + n16 / 4 of rows d = 4 i + kd; component
-//                  c of it is the A operand of product (i, c), whose row n16 is token TV x + c;
-//                  B is q[row n16][4 i + kd]. Lane l then holds, in s[c][v], the score of q row
-//                  n16 for token TV (4 v + kd) + c (output row 4 kd + v is lane row n16 = 4 kd +
-//                  v, whose vector is 4 v + kd).
-//   O += P . V     lane l loads vector 4 u + kd of rows d = 16 nb + n16; component c is the B
-//                  operand of product (u, c, nb), whose k slot kd is token TV (4 u + kd) + c: the
-//                  token of s[c][u], so A is that register as it stands.
+// consecutive tokens of one d. A tile is 16 vectors (64 or 128 tokens), vector x = tokens
+// TV x .. TV x + TV - 1. With lane l, kd = l / 16, n16 = l % 16:
+//   K: lane l loads vector 4 (n16 % 4) + n16 / 4 of rows d = 4 i + kd.
+//   V: lane l loads vectors 4 u + kd of rows d = 16 nb + n16.
 // Either load covers whole 128-byte lines: 4 consecutive K rows of each page (16-token pages:
 // 256 bytes per page in fp32, 128 in 16 bits), or 16 V rows of one page (two in 16 bits).
+//
+// fp32 storage, v_mfma_f32_16x16x4_f32 (A: lane l holds A[n16][kd]; B: B[kd][n16]; C: lane l
+// holds C[4 kd + v][n16]):
+//   S^T = K . Q^T  component c of K row i is the A operand of product (i, c), whose row n16 is
+//                  token TV x + c; B is q[row n16][4 i + kd]. Lane l then holds in s[c][v] the
+//                  score of q row n16 for token TV (4 v + kd) + c (output row 4 kd + v is lane
+//                  row n16 = 4 kd + v, whose vector is 4 v + kd).
+//   O += P . V     component c of V vector (u, nb) is the B operand of product (u, c, nb), whose
+//                  k slot kd is token TV (4 u + kd) + c: the token of s[c][u], so A is that
+//                  register as it stands.
+// 16-bit storage, v_mfma_f32_16x16x32 (A: lane l holds A[n16][8 kd .. + 7]; B: B[8 kd .. + 7][n16];
+// C as above), whose products of 16-bit values are exact in fp32:
+//   S^T = K . Q^T  k slot 8 kd + e of product (I, c) is row d = 4 (8 I + e) + kd, so A is
+//                  component c of the lane's K rows 8 I .. 8 I + 7 (four v_perm_b32) and B the
+//                  same elements of q row n16. The scores come out in the same places.
+//   O += P . V     a V vector is a whole B operand (k slot 8 kd + e is token 8 (4 u + kd) + e) and
+//                  A the eight probabilities s[0..7][u], as the sum of three 16-bit terms that
+//                  carry all 24 bits of an fp32 value (split3): three products instead of the
+//                  eight 16x16x4 ones that widened V would take, each of them half as long.
 #pragma once
 
 #include "attn_tiles.h"
@@ -35,15 +43,6 @@ struct Vec {
   using T = typename Elem<DT>::T;
   static constexpr int TV = 16 / int(sizeof(T));  // tokens of a 16-byte vector
   static constexpr int TOKENS = 16 * TV;          // tokens of a tile
-  // component c (compile-time after unrolling) of a vector, widened
-  __device__ __forceinline__ static float get(const uint4& x, int c) {
-    const uint32_t w = TV == 4 ? (c == 0 ? x.x : c == 1 ? x.y : c == 2 ? x.z : x.w)
-                               : (c < 2 ? x.x : c < 4 ? x.y : c < 6 ? x.z : x.w);
-    if constexpr (DT == PIA_DTYPE_F32) return __uint_as_float(w);
-    else if constexpr (DT == PIA_DTYPE_F16)
-      return half_to_f32(uint16_t((c & 1) ? (w >> 16) : (w & 0xffffu)));
-    else return (c & 1) ? bf16_hi(w) : bf16_lo(w);
-  }
   // components at or past n (n <= 0: all of them) become zero
   __device__ __forceinline__ static void keep_below(uint4& x, int n) {
     if constexpr (TV == 4) {
@@ -79,26 +78,90 @@ struct Vec {
     if constexpr (DT == PIA_DTYPE_F32) return __float_as_uint(*p);
     else return *p;
   }
-  __device__ __forceinline__ static float widen(uint32_t bits) {
-    if constexpr (DT == PIA_DTYPE_F32) return __uint_as_float(bits);
-    else if constexpr (DT == PIA_DTYPE_F16) return half_to_f32(uint16_t(bits));
-    else return bf16_lo(bits);
-  }
 };
 
 __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// scores += K . Q^T over N K vectors (rows 4 (i0 + i) + kd), q[i0 + i] the matching q elements
-template <int DT, int N, int QN>
-__device__ __forceinline__ void qk(const uint4 (&kr)[N], const float (&q)[QN], int i0,
+// component c (compile-time after unrolling) of an fp32 vector
+__device__ __forceinline__ float comp(const uint4& x, int c) {
+  return __uint_as_float(c == 0 ? x.x : c == 1 ? x.y : c == 2 ? x.z : x.w);
+}
+__device__ __forceinline__ uint32_t word(const uint4& x, int w) {
+  return w == 0 ? x.x : w == 1 ? x.y : w == 2 ? x.z : x.w;
+}
+
+// s += K . Q^T over the 16 K rows of kr; q: the lane's q elements of those rows in LDS (fp32: 16
+// floats; 16-bit: 16 raw elements), 16-byte aligned
+template <int DT>
+__device__ __forceinline__ void qk(const uint4 (&kr)[16], const void* q,
                                    f32x4_t (&s)[Vec<DT>::TV]) {
+  const uint4* qv = reinterpret_cast<const uint4*>(q);
+  if constexpr (DT == PIA_DTYPE_F32) {
 #pragma unroll
-  for (int i = 0; i < N; ++i)
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const uint4 x = qv[i4];
 #pragma unroll
-    for (int c = 0; c < Vec<DT>::TV; ++c)
-      s[c] = mfma_f32(Vec<DT>::get(kr[i], c), q[i0 + i], s[c]);
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          s[c] = mfma_f32(comp(kr[4 * i4 + j], c), comp(x, j), s[c]);
+    }
+  } else {
+#pragma unroll
+    for (int I = 0; I < 2; ++I) {
+      __builtin_amdgcn_sched_barrier(0);  // one q chunk and its operands at a time (registers)
+      const uint4 x = qv[I];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        uint32_t a[4];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+          const uint32_t r0 = word(kr[8 * I + 2 * f], c >> 1);
+          const uint32_t r1 = word(kr[8 * I + 2 * f + 1], c >> 1);
+          a[f] = __builtin_amdgcn_perm(r1, r0, (c & 1) ? 0x07060302u : 0x05040100u);
+        }
+        s[c] = tile::mfma16<DT>(make_uint4(a[0], a[1], a[2], a[3]), x, s[c]);
+      }
+    }
+  }
+}
+
+// 16-bit pair (pack16x2) back to fp32
+template <int DT>
+__device__ __forceinline__ float wide_lo(uint32_t x) {
+  if constexpr (DT == PIA_DTYPE_F16) return half_to_f32(uint16_t(x & 0xffffu));
+  else return bf16_lo(x);
+}
+template <int DT>
+__device__ __forceinline__ float wide_hi(uint32_t x) {
+  if constexpr (DT == PIA_DTYPE_F16) return half_to_f32(uint16_t(x >> 16));
+  else return bf16_hi(x);
+}
+
+// Eight fp32 values s[0..7][u] as three 16-bit operands whose sum they are: each term is what the
+// ones before leave, rounded to nearest. Three bf16 terms hold the 24 bits of any fp32 value that
+// is normal in all of them; three fp16 terms do for values of 2^-1 .. 2^15, below which the last
+// terms go denormal (the caller scales the probabilities by kSplitShift, so what is lost is under
+// 2^-39 of the largest).
+template <int DT>
+constexpr float kSplitShift = DT == PIA_DTYPE_F16 ? 15.f : 0.f;  // log2 units
+template <int DT>
+__device__ __forceinline__ void split3(const f32x4_t (&s)[8], int u, uint4 (&t)[3]) {
+  uint32_t w[3][4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    float a = s[2 * f][u], b = s[2 * f + 1][u];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w[k][f] = tile::pack16x2<DT>(a, b);
+      a -= wide_lo<DT>(w[k][f]);
+      b -= wide_hi<DT>(w[k][f]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) t[k] = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
 }
 
 // O += P . V over the V vectors u0 .. u0 + NU - 1 (vr[nb * NU + u - u0]), NB blocks of 16 d
@@ -106,12 +169,23 @@ template <int DT, int NB, int NU>
 __device__ __forceinline__ void pv(const uint4 (&vr)[NB * NU], const f32x4_t (&p)[Vec<DT>::TV],
                                    int u0, f32x4_t (&acc)[NB]) {
 #pragma unroll
-  for (int u = 0; u < NU; ++u)
+  for (int u = 0; u < NU; ++u) {
+    if constexpr (DT == PIA_DTYPE_F32) {
 #pragma unroll
-    for (int c = 0; c < Vec<DT>::TV; ++c)
+      for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        acc[nb] = mfma_f32(p[c][u0 + u], Vec<DT>::get(vr[nb * NU + u], c), acc[nb]);
+        for (int nb = 0; nb < NB; ++nb)
+          acc[nb] = mfma_f32(p[c][u0 + u], comp(vr[nb * NU + u], c), acc[nb]);
+    } else {
+      __builtin_amdgcn_sched_barrier(0);  // one set of terms at a time (registers)
+      uint4 t[3];
+      split3<DT>(p, u0 + u, t);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) acc[nb] = tile::mfma16<DT>(t[k], vr[nb * NU + u], acc[nb]);
+    }
+  }
 }
 
 // 16-byte non-temporal load (K / V read once per launch) or an ordinary one (read again by

@@ -18,11 +18,14 @@
 // 2. paged_decode_mfma<G> (G = 3, 5..8, 16): the same split, cursor, partials and merge, with
 //    the tile work of a step on the matrix cores (QK^T and PV as 16x16x32 MFMAs, K through a
 //    swizzled LDS tile and transposing reads, V straight into the MFMA operand registers).
-// 3. paged_attention_tiled<DT, C, VEC, R>: everything else up to head_dim 512 and G * head_dim
+// 3. paged_decode_f32<DT, D>: the same split, cursor, partials and merge with fp32 precision
+//    throughout, for fp32 pools, head_dim 64, other page sizes and group sizes up to 16, where
+//    the call brings scratch.
+// 4. paged_attention_tiled<DT, C, VEC, R>: everything else up to head_dim 512 and G * head_dim
 //    8192 (any dtype and page size, several query rows per sequence with optional causal
 //    offsets). One workgroup per (query row, kv head) serves its G q heads from K / V chunks of
 //    C keys staged once in LDS (described where it is defined).
-// 4. paged_attention_generic<DT, DPL>: what the tiled kernel's LDS or register budget does not
+// 5. paged_attention_generic<DT, DPL>: what the tiled kernel's LDS or register budget does not
 //    take (G * head_dim above 8192). One wave per (query row, head); keys are processed 64 at a
 //    time (lane = key for QK, lane = head-dim element for PV).
 #include <algorithm>
@@ -32,6 +35,7 @@
 #include <type_traits>
 
 #include "attn_tiles.h"
+#include "attn_tiles_f32.h"
 #include "pia_internal.h"
 
 namespace pia {
@@ -220,10 +224,10 @@ struct DecodeScratchLayout {
   int64_t part_offset;
   int64_t total_bytes;
 };
-constexpr DecodeScratchLayout decode_scratch_layout(int G, int waves) {
+constexpr DecodeScratchLayout decode_scratch_layout(int G, int waves, int D = FD_D) {
   return {(int64_t(waves) * 8 + 8 + 255) / 256 * 256,
           (int64_t(waves) * 8 + 8 + 255) / 256 * 256 +
-              int64_t(waves) * 2 * G * (FD_D + 2) * int64_t(sizeof(float))};
+              int64_t(waves) * 2 * G * (D + 2) * int64_t(sizeof(float))};
 }
 // Group sizes of the fast kernels: 1, 2, 4 on the vector ALU (paged_decode_stream), 3, 5..8 and 16
 // on the matrix cores (paged_decode_mfma, whose 16-row MFMA blocks hold up to 16 q rows).
@@ -322,28 +326,28 @@ __device__ __forceinline__ uint64_t* sd_counters(int32_t* ws_meta) {
   return reinterpret_cast<uint64_t*>((reinterpret_cast<uintptr_t>(ws_meta) + 7) & ~uintptr_t(7));
 }
 
-// Step prefix of the batch, built by every wave in its own LDS copy: seq_q[b] = steps of the
-// sequences before b (seq_q[B] = all of them), seq_len[b] = b's clamped context length (with
-// SD_NO_APPEND in append mode when its raw length does not fit its block table). Returns the
-// steps per kv head, sum_b ceil(L_b / 128).
-template <bool APPEND>
+// Step prefix of the batch, built by every wave in its own LDS copy: seq_q[b] = steps (of STEP
+// tokens) of the sequences before b (seq_q[B] = all of them), seq_len[b] = b's clamped context
+// length (with SD_NO_APPEND in append mode when its raw length does not fit its block table).
+// Returns the steps per kv head, sum_b ceil(L_b / STEP).
+template <bool APPEND, int STEP = SD_STEP_TOKENS>
 __device__ __forceinline__ int sd_build_prefix(const int32_t* __restrict__ context_lens, int B,
                                                int64_t bt_stride, int* seq_q, int* seq_len,
-                                               int lane) {
+                                               int lane, int P = FD_P) {
   constexpr int NCH = SD_MAX_SEQS / 64;
   int lv[NCH], lflag[NCH];
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     const int i = c * 64 + lane;
     const int raw = (c * 64 < B && i < B) ? context_lens[i] : 0;
-    lv[c] = clamp_len(raw, bt_stride, FD_P);
+    lv[c] = clamp_len(raw, bt_stride, P);
     lflag[c] = (APPEND && raw != lv[c]) ? SD_NO_APPEND : 0;
   }
   int carry = 0;
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     if (c * 64 >= B) break;
-    const int incl = wave_inclusive_scan((lv[c] + SD_STEP_TOKENS - 1) / SD_STEP_TOKENS, lane);
+    const int incl = wave_inclusive_scan((lv[c] + STEP - 1) / STEP, lane);
     const int i = c * 64 + lane;
     if (i < B) {
       seq_q[i + 1] = carry + incl;
@@ -357,12 +361,13 @@ __device__ __forceinline__ int sd_build_prefix(const int32_t* __restrict__ conte
 }
 
 // Rows of sequences with no steps are written as zeros: wave w takes sequences w, w + NW, ...
-__device__ __forceinline__ void sd_zero_empty_rows(uint16_t* out, const int* seq_len, int B,
-                                                   int Hq, int w, int NW, int lane) {
+template <int D = FD_D, typename T>
+__device__ __forceinline__ void sd_zero_empty_rows(T* out, const int* seq_len, int B, int Hq,
+                                                   int w, int NW, int lane) {
   for (int b = w; b < B; b += NW) {
     if ((uniform(seq_len[b]) & ~SD_NO_APPEND) == 0) {
-      uint16_t* o = out + int64_t(b) * Hq * FD_D;
-      for (int i = lane; i < Hq * FD_D; i += 64) o[i] = 0;
+      T* o = out + int64_t(b) * Hq * D;
+      for (int i = lane; i < Hq * D; i += 64) o[i] = T(0);
     }
   }
 }
@@ -443,15 +448,16 @@ __device__ __forceinline__ void sd_flush_appends(const int64_t (*rec)[2], int n_
 // Arrivals at the end of a wave's range: its partials (slot 0 / 1: arr_first = the segment's
 // first global step or -1, arr_ns its steps, arr_row = b * Hkv + h) are written; count them in
 // on their segments' counters and merge every segment whose last partial this is. Partial
-// layout per slot: G rows of [D unnormalised output, running max (log2 units), row sum].
-template <int G, int DT>
+// layout per slot: G rows of [D unnormalised output, running max (log2 units), row sum]; a merge
+// takes GB of them at a time.
+template <int GB, int DT, int D = FD_D>
 __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
                                                     const int (&arr_ns)[2],
                                                     const int (&arr_row)[2], int Dp, int Ce,
                                                     const float* ws_part, int32_t* ws_meta,
-                                                    uint64_t token, uint16_t* out, int Hkv,
-                                                    int lane) {
-  constexpr int D = FD_D;
+                                                    uint64_t token, typename Elem<DT>::T* out,
+                                                    int Hkv, int lane, int G = GB) {
+  constexpr int ND = D / 64;  // lane l: elements l + 64 i of every row
   if (arr_first[0] < 0 && arr_first[1] < 0) return;
   uint64_t* ctr = sd_counters(ws_meta);
   const int inc = Ce < Dp ? 1 : 2;  // odd waves hold no steps when pairs have one step
@@ -471,52 +477,63 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
   for (int k = 0; k < 2; ++k) {
     if (!merge[k]) continue;
     // one online pass over the pieces in wave order (slot 1 of the first wave, slot 0 of the
-    // rest); lane l: elements l and l + 64 of every row
+    // rest)
     const int c0 = stream_range_of(arr_first[k], Dp, Ce);
     const int c1 = stream_range_of(arr_first[k] + arr_ns[k] - 1, Dp, Ce);
-    float M[G], o0[G], o1[G], lt[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      M[g] = kNegBig;
-      o0[g] = o1[g] = lt[g] = 0.f;
-    }
-    // pieces eight (G <= 4) or four at a time: their loads in flight together, folded in order
-    constexpr int PB = G <= 4 ? 8 : 4;
-    for (int cb = c0; cb <= c1; cb += PB * inc) {
-      float mc[PB][G], lc[PB][G], a0[PB][G], a1[PB][G];
-#pragma unroll
-      for (int u = 0; u < PB; ++u) {
-        const int c = cb + u * inc;
-        if (c > c1) continue;
-        const float* pp = ws_part + (int64_t(c) * 2 + (c == c0 ? 1 : 0)) * G * (D + 2);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          mc[u][g] = sd_load(pp + g * (D + 2) + D);
-          lc[u][g] = sd_load(pp + g * (D + 2) + D + 1);
-          a0[u][g] = sd_load(pp + g * (D + 2) + lane);
-          a1[u][g] = sd_load(pp + g * (D + 2) + 64 + lane);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < PB; ++u) {
-        if (cb + u * inc > c1) continue;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const float mn = fmaxf(M[g], mc[u][g]);
-          const float fo = fast_exp2(M[g] - mn), fc = fast_exp2(mc[u][g] - mn);
-          lt[g] = lt[g] * fo + lc[u][g] * fc;
-          o0[g] = o0[g] * fo + a0[u][g] * fc;
-          o1[g] = o1[g] * fo + a1[u][g] * fc;
-          M[g] = mn;
-        }
-      }
-    }
     const int b = arr_row[k] / Hkv, h = arr_row[k] - b * Hkv;
-    uint16_t* orow = out + (int64_t(b) * Hkv * G + int64_t(h) * G) * D;
+    typename Elem<DT>::T* orow = out + (int64_t(b) * Hkv * G + int64_t(h) * G) * D;
+    for (int g0 = 0; g0 < G; g0 += GB) {
+      float M[GB], o[GB][ND], lt[GB];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      orow[g * D + lane] = to16<DT>(lt[g] > 0.f ? o0[g] / lt[g] : 0.f);
-      orow[g * D + 64 + lane] = to16<DT>(lt[g] > 0.f ? o1[g] / lt[g] : 0.f);
+      for (int g = 0; g < GB; ++g) {
+        M[g] = -INFINITY;
+        lt[g] = 0.f;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) o[g][i] = 0.f;
+      }
+      // pieces eight (GB <= 4), four or two at a time: their loads in flight together, folded
+      // in order
+      constexpr int PB = GB <= 4 ? 8 : GB <= 8 ? 4 : 2;
+      for (int cb = c0; cb <= c1; cb += PB * inc) {
+        float mc[PB][GB], lc[PB][GB], a[PB][GB][ND];
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+          const int c = cb + u * inc;
+          if (c > c1) continue;
+          const float* pp = ws_part + ((int64_t(c) * 2 + (c == c0 ? 1 : 0)) * G + g0) * (D + 2);
+#pragma unroll
+          for (int g = 0; g < GB; ++g) {
+            if (g0 + g >= G) continue;
+            mc[u][g] = sd_load(pp + g * (D + 2) + D);
+            lc[u][g] = sd_load(pp + g * (D + 2) + D + 1);
+#pragma unroll
+            for (int i = 0; i < ND; ++i) a[u][g][i] = sd_load(pp + g * (D + 2) + 64 * i + lane);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+          if (cb + u * inc > c1) continue;
+#pragma unroll
+          for (int g = 0; g < GB; ++g) {
+            if (g0 + g >= G) continue;
+            const float mn = fmaxf(M[g], mc[u][g]);
+            const float fo = M[g] == mn ? 1.f : fast_exp2(M[g] - mn);
+            const float fc = mc[u][g] == mn ? 1.f : fast_exp2(mc[u][g] - mn);
+            lt[g] = lt[g] * fo + lc[u][g] * fc;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) o[g][i] = o[g][i] * fo + a[u][g][i] * fc;
+            M[g] = mn;
+          }
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < GB; ++g) {
+        if (g0 + g >= G) continue;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+          Elem<DT>::store(orow, int64_t(g0 + g) * D + 64 * i + lane,
+                          lt[g] > 0.f ? o[g][i] / lt[g] : 0.f);
+      }
     }
   }
 }
@@ -1406,6 +1423,398 @@ __global__ __launch_bounds__(64, 1) void paged_decode_mfma(
 }
 
 // ---------------------------------------------------------------------------------------------
+// Stream decode kernel with fp32 precision throughout, on the matrix cores: any storage type
+// (fp32, fp16, bf16), head_dim 64 or 128, page sizes that are whole 16-byte vectors, up to 16 q
+// rows per kv head, for the shapes the two 16-bit kernels above do not take.
+//
+// The work split, cursor, partial slots, arrivals and merge are paged_decode_stream's, with steps
+// of one tile (64 fp32 or 128 16-bit tokens), two waves per SIMD. K and V go from memory straight
+// into MFMA operands (attn_tiles_f32.h): 16x16x4 products of fp32 pools, or 16x16x32 ones of
+// 16-bit pools with the fp32 probabilities in three 16-bit terms. HBM-bound: the products of an
+// fp32 tile take 32 D cycles on each of four SIMDs at two waves, about a third of the time in
+// which HBM delivers the tile; those of a 16-bit tile an eighth of that. (Widening 16-bit K / V to
+// 16x16x4 products instead: twice the cycles of fp32 per byte, 74.0 us for the second size below.)
+// Pipeline, two register buffers of 16 vectors (16 KiB each):
+//   D = 128  A, B: the tile's K rows 0..63, 64..127.
+//            QK(A) | issue V u 0,1 -> A | QK(B) | softmax | issue V u 2,3 -> B | PV(A) |
+//            issue next K -> A | PV(B) | issue next K -> B
+//   D = 64   A: the tile's K, B: its V.  QK(A) | issue next K -> A | softmax | PV(B) |
+//            issue next V -> B
+// Block-table entries are fetched two steps ahead, before the step's tile loads: vector memory
+// counters retire in order, so a wait on them then holds for no tile load behind them.
+// Measured against paged_attention_tiled, which served these shapes (whole calls with the KV
+// append): 32 sequences of 1..2048 tokens, 16/8 heads of 128, fp32: 358.4 -> 59.7 us (4.4 TB/s); 48 of
+// 256..4096, 32/8 heads of 64, bf16: 471.0 -> 55.6 us (4.1 TB/s).
+// ---------------------------------------------------------------------------------------------
+template <int DT, int D, bool APPEND>
+__global__ __launch_bounds__(64, 2) void paged_decode_f32(
+    typename Elem<DT>::T* __restrict__ out, const typename Elem<DT>::T* __restrict__ q,
+    int64_t q_seq_stride, const typename Elem<DT>::T* kpool, const typename Elem<DT>::T* vpool,
+    const int32_t* __restrict__ block_tables, int64_t bt_stride,
+    const int32_t* __restrict__ context_lens, int B, int Hkv, int G, int P, int64_t num_pages,
+    float* __restrict__ ws_part, int32_t* __restrict__ ws_meta, float scale_log2,
+    typename Elem<DT>::T* kpool_w, typename Elem<DT>::T* vpool_w,
+    const typename Elem<DT>::T* __restrict__ k_new,
+    const typename Elem<DT>::T* __restrict__ v_new, int64_t new_seq_stride, uint64_t token) {
+  using tile::f32x4_t;
+  using V = tile32::Vec<DT>;
+  using T = typename Elem<DT>::T;
+  static_assert(D == 64 || D == 128, "two register buffers of 16 vectors");
+  constexpr int TV = V::TV, STEP = V::TOKENS, NB = D / 16, NI = D / 4;
+  constexpr int NU = D == 128 ? 2 : 4;       // V vectors u of one buffer
+  constexpr int QS = NI + 16 / int(sizeof(T));  // LDS stride of a lane's q elements (bank skew)
+  constexpr int ND = D / 64;
+  const int lane = threadIdx.x, w = blockIdx.x, NW = gridDim.x;
+  // l / 16 and l % 16, recomputed at each use: what is derived from them would otherwise be kept
+  // across the loop and spilled, and the reload of a spilled register waits for every tile load
+  // issued before it
+  auto lane_now = [&]() -> int {
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  const int Hq = Hkv * G;
+  extern __shared__ int sd_lds[];
+  int* seq_q = sd_lds;            // [B + 1]: steps of the sequences before b
+  int* seq_len = sd_lds + B + 1;  // [B]: clamped context length
+  // [lane]: q[n16][4 i + kd]: fp32 pre-scaled, 16-bit as given (the scores are scaled). Read from
+  // LDS for every tile: in registers it does not fit two waves per SIMD beside the buffers.
+  __shared__ __align__(16) T qs[64 * QS];
+  __shared__ uint32_t new_lds[APPEND ? 2 * D : 1];  // raw elements of k_new, v_new
+  // append mode: deferred new-token stores, {pool element offset of the slot, k_new offset}
+  __shared__ int64_t app_rec[APPEND ? SD_APP_REC : 1][2];
+  int n_rec = 0;
+
+  const int T_all =
+      Hkv * sd_build_prefix<APPEND, STEP>(context_lens, B, bt_stride, seq_q, seq_len, lane, P);
+  const int Dp = stream_pair_steps(T_all, NW), Ce = stream_even_share(Dp);
+  sd_zero_empty_rows<D>(out, seq_len, B, Hq, w, NW, lane);
+  const int start = (w >> 1) * Dp + ((w & 1) ? Ce : 0);
+  const int end = min((w >> 1) * Dp + ((w & 1) ? Dp : Ce), T_all);
+  if (start >= end) return;
+  const int span = end - start;
+  const StreamPlan plan{seq_q, seq_len, B, Hkv, APPEND};
+
+  // The tile's vector x = lane % 16 (tokens TV x ..): its page id, its element offset inside the
+  // pool (row d = 0 of the head's tile) and its valid tokens. Vectors past the sequence repeat
+  // its last page; ids outside the pool read page 0 and hold no key.
+  const int vpp = P / TV;  // vectors per page row
+  auto load_bt = [&](const StreamCursor& c) -> int {
+    const int npg = (c.L + P - 1) / P, n16 = lane_now() & 15;
+    return block_tables[int64_t(c.b) * bt_stride + min((c.ls * 16 + n16) / vpp, npg - 1)];
+  };
+  auto id_ok = [&](int id) { return id >= 0 && int64_t(id) < num_pages; };
+  auto vec_off = [&](const StreamCursor& c, int id) -> int64_t {
+    const int x = c.ls * 16 + (lane_now() & 15);
+    return (int64_t(id_ok(id) ? id : 0) * Hkv + c.h) * D * P + (x % vpp) * TV;
+  };
+  auto shfl64 = [](int64_t v, int src) -> int64_t {
+    const int lo = __shfl(int(v), src, 64), hi = __shfl(int(v >> 32), src, 64);
+    return (int64_t(hi) << 32) | uint32_t(lo);
+  };
+  const int64_t P4 = 4 * int64_t(P), P16 = 16 * int64_t(P);
+  // K rows 4 (i0 + i) + kd of vector 4 (n16 % 4) + n16 / 4
+  auto load_k = [&](uint4 (&kr)[16], int64_t off, int i0) {
+    const int l = lane_now(), kd = l >> 4, n16 = l & 15;
+    const T* p = kpool + shfl64(off, 4 * (n16 & 3) + (n16 >> 2)) + (4 * i0 + kd) * int64_t(P);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) kr[i] = tile32::load16<true>(p + i * P4);
+  };
+  // V rows 16 nb + n16 of vectors 4 (u0 + u) + kd
+  auto load_v = [&](uint4 (&vr)[16], int64_t off, int u0) {
+    const int l = lane_now(), kd = l >> 4, n16 = l & 15;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const T* p = vpool + shfl64(off, 4 * (u0 + u) + kd) + n16 * int64_t(P);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) vr[nb * NU + u] = tile32::load16<true>(p + nb * P16);
+    }
+  };
+  // a segment's G * D q values into qs, and a new token's rows into new_lds (raw elements)
+  auto stage_q = [&](const StreamCursor& c) {
+    const T* p = q + int64_t(c.b) * q_seq_stride + int64_t(c.h) * G * D;
+    for (int e = lane; e < G * D; e += 64) {
+      const int g = e / D, d = e % D;
+      if constexpr (DT == PIA_DTYPE_F32)
+        qs[((d & 3) * 16 + g) * QS + (d >> 2)] = p[e] * scale_log2;
+      else
+        qs[((d & 3) * 16 + g) * QS + (d >> 2)] = p[e];
+    }
+  };
+  auto stage_new = [&](int64_t src) {
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      new_lds[lane + 64 * i] = V::raw(k_new + src + lane + 64 * i);
+      new_lds[D + lane + 64 * i] = V::raw(v_new + src + lane + 64 * i);
+    }
+  };
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto is_app = [&](const StreamCursor& c) { return APPEND && c.app && c.ls == c.ns - 1; };
+  auto new_src = [&](const StreamCursor& c) {
+    return int64_t(c.b) * new_seq_stride + int64_t(c.h) * D;
+  };
+
+  float m = -INFINITY, lsum = 0.f;  // of q row n16 (lsum: this lane's scores only)
+  f32x4_t acc[NB];                  // rows 4 kd + j, column 16 nb + n16
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  int gs = start;
+  StreamCursor cur = plan.seg_of(gs);
+  StreamCursor nxt = gs + 1 < end ? plan.next_of(cur) : cur;
+  // partials this wave writes (slot 0, slot 1): the first global step, step count and row of
+  // their segments, for the arrivals after the range (arr_first -1: no partial in that slot)
+  int arr_first[2] = {-1, -1}, arr_ns[2] = {0, 0}, arr_row[2] = {0, 0};
+  uint4 bufA[16], bufB[16];
+  int bt_cur = load_bt(cur), bt_nxt = load_bt(nxt);
+  int64_t off_cur;
+  {
+    SegmentCounters counters;
+    counters.begin(plan, cur, start, end, Dp, Ce, ws_meta, lane);
+    off_cur = vec_off(cur, bt_cur);
+    load_k(bufA, off_cur, 0);
+    if constexpr (D == 128) load_k(bufB, off_cur, 16);
+    else load_v(bufB, off_cur, 0);
+    counters.finish(token, lane);
+    for (int i = lane; i < 64 * QS; i += 64) qs[i] = T(0);  // rows G..15 stay zero
+    wave_sync();
+    stage_q(cur);
+    wave_sync();
+  }
+
+  for (;;) {
+    {  // issue priority from progress: quartile 0 of the range -> 3, quartile 3 -> 0
+      const int quarter = (4 * (gs - start)) / span;
+      if (quarter <= 0) __builtin_amdgcn_s_setprio(3);
+      else if (quarter == 1) __builtin_amdgcn_s_setprio(2);
+      else if (quarter == 2) __builtin_amdgcn_s_setprio(1);
+      else __builtin_amdgcn_s_setprio(0);
+    }
+    const bool has_next = gs + 1 < end;
+    const StreamCursor far = gs + 2 < end ? plan.next_of(nxt) : nxt;
+    const int bt_far = load_bt(far);
+    const bool app_step = is_app(cur);
+    const int tn = min(STEP, cur.L - cur.ls * STEP) - 1;  // the new token of an append step
+    // valid tokens of vector n16, and on masked steps those of the lane's vectors 4 v + kd
+    const int nv16 = id_ok(bt_cur) ? cur.L - (cur.ls * 16 + (lane_now() & 15)) * TV : 0;
+    const bool masked = __ballot(nv16 < TV) != 0;
+    const int64_t off_nxt = vec_off(nxt, bt_nxt);
+    // a segment's q when it opens, the new token at its end: once per segment, behind the K loads
+    // in flight (kept in registers from a step ahead they cost the tile buffers their room)
+    if ((cur.ls == 0 && gs > start) || (APPEND && app_step)) {
+      wave_sync();  // the previous step's LDS reads are done
+      if (cur.ls == 0 && gs > start) stage_q(cur);
+      if (APPEND && app_step) stage_new(new_src(cur));
+      wave_sync();
+    }
+
+    auto put_k = [&](uint4 (&kr)[16], int i0) {
+      if (APPEND && app_step) {
+        const int l = lane_now(), kd = l >> 4, n16 = l & 15;
+        const bool own = 4 * (n16 & 3) + (n16 >> 2) == tn / TV;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          V::put(kr[i], tn % TV, new_lds[4 * (i0 + i) + kd], own);
+      }
+    };
+    auto put_v = [&](uint4 (&vr)[16], int u0) {
+      if (APPEND && app_step) {
+        const int l = lane_now(), kd = l >> 4, n16 = l & 15;
+        const int xn = tn / TV;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const uint32_t x = new_lds[D + 16 * nb + n16];
+#pragma unroll
+          for (int u = 0; u < NU; ++u) V::put(vr[nb * NU + u], tn % TV, x, 4 * (u0 + u) + kd == xn);
+        }
+      }
+    };
+    // V components that are no keys -> 0 (stale memory may hold non-finite values)
+    auto mask_v = [&](uint4 (&vr)[16], int u0) {
+      if (masked) {
+        const int kd = lane_now() >> 4;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          const int n = __shfl(nv16, 4 * (u0 + u) + kd, 64);
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) V::keep_below(vr[nb * NU + u], n);
+        }
+      }
+    };
+
+    f32x4_t s[TV];
+#pragma unroll
+    for (int c = 0; c < TV; ++c) s[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_sched_barrier(0);
+    put_k(bufA, 0);
+    tile32::qk<DT>(bufA, &qs[lane_now() * QS], s);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (D == 128) {
+      load_v(bufA, off_cur, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      put_k(bufB, 16);
+      tile32::qk<DT>(bufB, &qs[lane_now() * QS + 16], s);
+    } else {
+      if (has_next) load_k(bufA, off_nxt, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // softmax of q row n16: token TV (4 v + kd) + c of the tile is s[c][v]
+    if constexpr (DT != PIA_DTYPE_F32) {
+#pragma unroll
+      for (int c = 0; c < TV; ++c) s[c] *= scale_log2;
+    }
+    if (masked) {
+      const int kd = lane_now() >> 4;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int n = __shfl(nv16, 4 * v + kd, 64);
+#pragma unroll
+        for (int c = 0; c < TV; ++c) s[c][v] = c < n ? s[c][v] : -INFINITY;
+      }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int c = 0; c < TV; ++c)
+      mx = fmaxf(mx, fmaxf(fmaxf(s[c][0], s[c][1]), fmaxf(s[c][2], s[c][3])));
+    const float mn = fmaxf(m, tile::max_col4(mx));
+    // a row with no key yet: p = 2^-inf = 0
+    const float nm = mn == -INFINITY ? 0.f : mn - tile32::kSplitShift<DT>;
+    const bool moved = m != mn;
+    const float alpha = moved ? fast_exp2(m - mn) : 1.f;
+    m = mn;
+    float ps = 0.f;
+#pragma unroll
+    for (int c = 0; c < TV; ++c) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s[c][v] = fast_exp2(s[c][v] - nm);
+      ps += (s[c][0] + s[c][1]) + (s[c][2] + s[c][3]);
+    }
+    lsum = lsum * alpha + ps;
+    if (__ballot(moved)) {
+      const int kd = lane_now() >> 4;
+      float aj[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) aj[j] = __shfl(alpha, 4 * kd + j, 64);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[nb][j] *= aj[j];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (D == 128) {
+      load_v(bufB, off_cur, 2);
+      __builtin_amdgcn_sched_barrier(0);
+      put_v(bufA, 0);
+      mask_v(bufA, 0);
+      tile32::pv<DT, NB, NU>(bufA, s, 0, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (has_next) load_k(bufA, off_nxt, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      put_v(bufB, 2);
+      mask_v(bufB, 2);
+      tile32::pv<DT, NB, NU>(bufB, s, 2, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (has_next) load_k(bufB, off_nxt, 16);
+    } else {
+      put_v(bufB, 0);
+      mask_v(bufB, 0);
+      tile32::pv<DT, NB, NU>(bufB, s, 0, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (has_next) load_v(bufB, off_nxt, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    if (APPEND && app_step) {  // the new token goes into its slot after the range
+      const int idn = __builtin_amdgcn_readlane(bt_cur, tn / TV);
+      if (id_ok(idn)) {
+        const int pos = cur.ls * STEP + tn;
+        const int64_t slot = (int64_t(idn) * Hkv + cur.h) * D * P + pos % P;
+        if (n_rec < SD_APP_REC) {
+          if (lane == 0) {
+            app_rec[n_rec][0] = slot;
+            app_rec[n_rec][1] = new_src(cur);
+          }
+          ++n_rec;
+        } else {
+#pragma unroll
+          for (int i = 0; i < ND; ++i) {
+            const int d = lane + 64 * i;
+            __builtin_nontemporal_store(k_new[new_src(cur) + d], kpool_w + slot + int64_t(d) * P);
+            __builtin_nontemporal_store(v_new[new_src(cur) + d], vpool_w + slot + int64_t(d) * P);
+          }
+        }
+      }
+    }
+
+    const bool seg_last = cur.ls == cur.ns - 1;
+    if (seg_last || !has_next) {
+      const float l_row = tile32::sum_col4(lsum);
+      const int l = lane_now(), kd = l >> 4, n16 = l & 15;
+      const int seg_first = gs - cur.ls;  // global index of the segment's first step
+      const int64_t row0 = int64_t(cur.b) * Hq + int64_t(cur.h) * G;
+      if (seg_last && seg_first >= start) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float lj = __shfl(l_row, 4 * kd + j, 64);
+          if (4 * kd + j >= G) continue;
+          const float inv = lj > 0.f ? 1.f / lj : 0.f;
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            Elem<DT>::store(out, (row0 + 4 * kd + j) * D + 16 * nb + n16, acc[nb][j] * inv);
+        }
+      } else {
+        const int slot = seg_first < start ? 0 : 1;
+        arr_first[slot] = seg_first;
+        arr_ns[slot] = cur.ns;
+        arr_row[slot] = cur.b * Hkv + cur.h;
+        // device-coherent partial stores (see paged_decode_stream)
+        float* part = ws_part + (int64_t(w) * 2 + slot) * G * (D + 2);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (4 * kd + j >= G) continue;
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            sd_store(part + (4 * kd + j) * (D + 2) + 16 * nb + n16, acc[nb][j]);
+        }
+        if (kd == 0 && n16 < G) {
+          sd_store(part + n16 * (D + 2) + D, m);
+          sd_store(part + n16 * (D + 2) + D + 1, l_row);
+        }
+      }
+      m = -INFINITY;
+      lsum = 0.f;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    if (!has_next) break;
+    cur = nxt;
+    nxt = far;
+    bt_cur = bt_nxt;
+    bt_nxt = bt_far;
+    off_cur = off_nxt;
+    ++gs;
+  }
+  sd_arrive_and_merge<4, DT, D>(arr_first, arr_ns, arr_row, Dp, Ce, ws_part, ws_meta, token, out,
+                                 Hkv, lane, G);
+  if constexpr (APPEND) {
+    wave_sync();
+    for (int r = 0; r < n_rec; ++r) {
+      const int64_t slot = app_rec[r][0], src = app_rec[r][1];
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        const int d = lane + 64 * i;
+        __builtin_nontemporal_store(k_new[src + d], kpool_w + slot + int64_t(d) * P);
+        __builtin_nontemporal_store(v_new[src + d], vpool_w + slot + int64_t(d) * P);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // General kernel
 // ---------------------------------------------------------------------------------------------
 template <int DT, int DPL>
@@ -2016,6 +2425,92 @@ int launch_stream_decode(int dtype, void* out, const void* q, int64_t q_seq_stri
                 s, k_new, v_new, new_seq_stride);
 }
 
+// Waves of a paged_decode_f32 launch: two single-wave workgroups per SIMD.
+int f32_waves() {
+  return std::max(2, std::min(device_cus() * SD_WAVES_PER_CU, SD_MAX_WAVES) & ~1);
+}
+
+// Scratch of paged_decode_f32 (0: not one of its shapes). It takes what the two 16-bit kernels do
+// not: head_dim 64 or 128, up to 16 q rows per kv head (one MFMA operand block), pages of whole
+// 16-byte vectors. Other shapes, and calls that bring no scratch, stay on the tiled kernel.
+int64_t f32_scratch_bytes(int dtype, int Hq, int Hkv, int D, int P) {
+  const int vec = dtype == PIA_DTYPE_F32 ? 4 : 8;
+  const int G = Hq / Hkv;
+  if (fast_path(dtype, Hq, Hkv, D, P) || (D != 64 && D != 128) || G > 16 || P % vec) return 0;
+  return decode_scratch_layout(G, f32_waves(), D).total_bytes;
+}
+
+// paged_decode_f32 for a call with scratch, if it takes it: *taken says whether it was launched
+// (or failed); otherwise nothing is enqueued. Sequences in launches of SD_MAX_SEQS, as above.
+template <int DT>
+int try_f32_decode_dt(bool* taken, void* out, const void* q, int64_t q_seq_stride,
+                      const void* k_pages, const void* v_pages, const int32_t* block_tables,
+                      int64_t bt_stride, const int32_t* context_lens, int num_seqs, int num_heads,
+                      int num_kv_heads, int D, int P, int64_t num_pages, float scale_log2,
+                      void* workspace, int64_t workspace_bytes, hipStream_t s, const void* k_new,
+                      const void* v_new, int64_t new_seq_stride) {
+  using T = typename Elem<DT>::T;
+  *taken = false;
+  const int64_t need = f32_scratch_bytes(DT, num_heads, num_kv_heads, D, P);
+  const int NW = f32_waves(), G = num_heads / num_kv_heads;
+  if (need == 0 || !workspace || workspace_bytes < need || !aligned(workspace, 4) ||
+      !aligned(k_pages, 16) || !aligned(v_pages, 16))
+    return 0;
+  // int32 step arithmetic, as for the 16-bit kernels; block tables beyond it stay on the tiled one
+  const int64_t steps = bt_stride > (int64_t(1) << 31) / P
+                            ? int64_t(1) << 31
+                            : ceil_div(bt_stride * P, tile32::Vec<DT>::TOKENS);
+  if (int64_t(num_kv_heads) * std::min(num_seqs, SD_MAX_SEQS) * steps + 2 * int64_t(NW) >=
+      (int64_t(1) << 31))
+    return 0;
+  *taken = true;
+  unsigned char* scratch = static_cast<unsigned char*>(workspace);
+  int32_t* ws_meta = reinterpret_cast<int32_t*>(scratch);
+  float* ws_part = reinterpret_cast<float*>(scratch + decode_scratch_layout(G, NW, D).part_offset);
+  T* kw = const_cast<T*>(reinterpret_cast<const T*>(k_pages));
+  T* vw = const_cast<T*>(reinterpret_cast<const T*>(v_pages));
+  for (int b0 = 0; b0 < num_seqs; b0 += SD_MAX_SEQS) {
+    const int Bs = std::min(SD_MAX_SEQS, num_seqs - b0);
+    T* o = reinterpret_cast<T*>(out) + int64_t(b0) * num_heads * D;
+    const T* qq = reinterpret_cast<const T*>(q) + int64_t(b0) * q_seq_stride;
+    const int32_t* bt = block_tables + int64_t(b0) * bt_stride;
+    const T* kn =
+        k_new ? reinterpret_cast<const T*>(k_new) + int64_t(b0) * new_seq_stride : nullptr;
+    const T* vn =
+        k_new ? reinterpret_cast<const T*>(v_new) + int64_t(b0) * new_seq_stride : nullptr;
+    const size_t lds = size_t(2 * Bs + 1) * sizeof(int32_t);
+    const uint64_t token = next_stream_token();
+#define PIA_F32(DD, AP)                                                                    \
+  hipLaunchKernelGGL((paged_decode_f32<DT, DD, AP>), dim3(unsigned(NW)), dim3(64), lds, s, \
+                     o, qq, q_seq_stride, (const T*)k_pages, (const T*)v_pages, bt, bt_stride, \
+                     context_lens + b0, Bs, num_kv_heads, G, P, num_pages, ws_part, ws_meta,   \
+                     scale_log2, kw, vw, kn, vn, new_seq_stride, token)
+    if (D == 128) {
+      if (kn) PIA_F32(128, true); else PIA_F32(128, false);
+    } else {
+      if (kn) PIA_F32(64, true); else PIA_F32(64, false);
+    }
+#undef PIA_F32
+    if (int rc = check_launch("paged_decode_f32")) return rc;
+  }
+  return 0;
+}
+
+int try_f32_decode(bool* taken, int dtype, void* out, const void* q, int64_t q_seq_stride,
+                   const void* k_pages, const void* v_pages, const int32_t* block_tables,
+                   int64_t bt_stride, const int32_t* context_lens, int num_seqs, int num_heads,
+                   int num_kv_heads, int D, int P, int64_t num_pages, float scale_log2,
+                   void* workspace, int64_t workspace_bytes, hipStream_t s,
+                   const void* k_new = nullptr, const void* v_new = nullptr,
+                   int64_t new_seq_stride = 0) {
+  auto* launch = dtype == PIA_DTYPE_F32   ? &try_f32_decode_dt<PIA_DTYPE_F32>
+                 : dtype == PIA_DTYPE_F16 ? &try_f32_decode_dt<PIA_DTYPE_F16>
+                                          : &try_f32_decode_dt<PIA_DTYPE_BF16>;
+  return launch(taken, out, q, q_seq_stride, k_pages, v_pages, block_tables, bt_stride,
+                context_lens, num_seqs, num_heads, num_kv_heads, D, P, num_pages, scale_log2,
+                workspace, workspace_bytes, s, k_new, v_new, new_seq_stride);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Library-owned scratch for pia_paged_decode_attention_noalloc: the meta ints (arrival
 // counters), then the wave partials, in one static device array per GPU (held until the process
@@ -2068,6 +2563,14 @@ extern "C" int64_t pia_paged_decode_workspace_bytes(int num_seqs, int num_heads,
   return decode_scratch_layout(G, SD_MAX_WAVES).total_bytes;
 }
 
+extern "C" int64_t pia_paged_decode_split_scratch_bytes(int num_heads, int num_kv_heads,
+                                                        int head_dim, int page_size, int dtype) {
+  if (num_heads <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads || page_size <= 0 ||
+      (dtype != PIA_DTYPE_F32 && dtype != PIA_DTYPE_F16 && dtype != PIA_DTYPE_BF16))
+    return 0;
+  return f32_scratch_bytes(dtype, num_heads, num_kv_heads, head_dim, page_size);
+}
+
 extern "C" int pia_paged_decode_scratch_layout(int num_heads, int num_kv_heads, int waves,
                                                int64_t* partials_offset, int64_t* total_bytes) {
   if (!partials_offset || !total_bytes) return fail(PIA_EINVAL, "decode_scratch_layout: null pointer");
@@ -2111,6 +2614,12 @@ extern "C" int pia_paged_decode_attention(void* out, const void* q, int64_t q_se
                                 num_pages, scale_log2, static_cast<unsigned char*>(workspace),
                                 SD_MAX_WAVES, s);
   }
+  bool taken = false;
+  if (int rc = try_f32_decode(&taken, dtype, out, q, q_seq_stride, k_pages, v_pages, block_tables,
+                              bt_stride, context_lens, num_seqs, num_heads, num_kv_heads, head_dim,
+                              page_size, num_pages, scale_log2, workspace, workspace_bytes, s))
+    return rc;
+  if (taken) return 0;
   return launch_generic_any(dtype, out, q, q_seq_stride, k_pages, v_pages, block_tables,
                             bt_stride, context_lens, nullptr, nullptr, num_seqs, num_seqs,
                             num_heads, num_kv_heads, head_dim, page_size, num_pages, scale_log2,
@@ -2150,6 +2659,13 @@ extern "C" int pia_paged_decode_append_attention(
                                 num_pages, scale_log2, static_cast<unsigned char*>(workspace),
                                 SD_MAX_WAVES, s, k_new, v_new, new_seq_stride);
   }
+  bool taken = false;
+  if (int rc = try_f32_decode(&taken, dtype, out, q, q_seq_stride, k_pages, v_pages, block_tables,
+                              bt_stride, context_lens, num_seqs, num_heads, num_kv_heads, head_dim,
+                              page_size, num_pages, scale_log2, workspace, workspace_bytes, s,
+                              k_new, v_new, new_seq_stride))
+    return rc;
+  if (taken) return 0;
   // any other shape: the new tokens into their slots, then the decode over the pool
   if (int rc = launch_kv_append(dtype, k_pages, v_pages, k_new, v_new, new_seq_stride,
                                 block_tables, bt_stride, context_lens, num_seqs, num_kv_heads,

@@ -33,6 +33,7 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "pia_kv_pages_chunks_copy": (_I, [_P, _I, _P, _P, _I, _I, _I, _I, _I, _L, _I, _I, _P]),
     "pia_paged_decode_workspace_bytes": (_L, [_I, _I, _I, _I, _I, _L]),
     "pia_paged_decode_scratch_layout": (_I, [_I, _I, _I, _P, _P]),
+    "pia_paged_decode_split_scratch_bytes": (_L, [_I, _I, _I, _I, _I]),
     "pia_paged_decode_attention": (
         _I, [_P, _P, _L, _P, _P, _P, _L, _P, _I, _I, _I, _I, _I, _L, _F, _I, _P, _L, _P]),
     "pia_paged_decode_append_attention": (

@@ -115,6 +115,23 @@ def decode_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, hea
                    head_dim, page_size, max_pages_per_seq)
 
 
+def _decode_scratch(q: torch.Tensor, Hkv: int, P: int, max_pages: int,
+                    workspace: torch.Tensor | None) -> tuple[torch.Tensor | None, int]:
+    """(workspace, its bytes) of a decode call: the caller's where it is large enough for the
+    call's kernel, else one allocated for the call; (None, 0) where no kernel takes one."""
+    B, Hq, D = q.shape
+    need = decode_workspace_bytes(B, Hq, Hkv, D, P, max_pages)
+    if not need:
+        need = N.query("pia_paged_decode_split_scratch_bytes", Hq, Hkv, D, P,
+                       N.dtype_code(q.dtype))
+    if not need:
+        return None, 0
+    have = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    if have < need:
+        return torch.empty(need, dtype=torch.uint8, device=q.device), need
+    return workspace, have
+
+
 def paged_decode_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                            block_tables: torch.Tensor, context_lens: torch.Tensor,
                            scale: float | None = None, out: torch.Tensor | None = None,
@@ -145,15 +162,12 @@ def paged_decode_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
         raise ValueError("out must be a contiguous [B, Hq, D] tensor of q's dtype")
     if B == 0:
         return out
-    need = decode_workspace_bytes(B, Hq, Hkv, D, P, block_tables.shape[1])
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+    workspace, ws_bytes = _decode_scratch(q, Hkv, P, block_tables.shape[1], workspace)
     scale = (1.0 / math.sqrt(D)) if scale is None else float(scale)
     N.call("pia_paged_decode_attention", out.data_ptr(), q.data_ptr(), q.stride(0),
            k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
            context_lens.data_ptr(), B, Hq, Hkv, D, P, num_pages, scale, N.dtype_code(q.dtype),
-           N.ptr(workspace) if need else None,
-           (workspace.numel() * workspace.element_size()) if need else 0, N.stream_of(dev))
+           N.ptr(workspace), ws_bytes, N.stream_of(dev))
     return out
 
 
@@ -197,16 +211,13 @@ def paged_decode_append_attention(q: torch.Tensor, k_pages: torch.Tensor, v_page
         raise ValueError("out must be a contiguous [B, Hq, D] tensor of q's dtype")
     if B == 0:
         return out
-    need = decode_workspace_bytes(B, Hq, Hkv, D, P, block_tables.shape[1])
-    if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+    workspace, ws_bytes = _decode_scratch(q, Hkv, P, block_tables.shape[1], workspace)
     scale = (1.0 / math.sqrt(D)) if scale is None else float(scale)
     N.call("pia_paged_decode_append_attention", out.data_ptr(), q.data_ptr(), q.stride(0),
            k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
            context_lens.data_ptr(), k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), B, Hq,
            Hkv, D, P, num_pages, scale, N.dtype_code(q.dtype),
-           N.ptr(workspace) if need else None,
-           (workspace.numel() * workspace.element_size()) if need else 0, N.stream_of(dev))
+           N.ptr(workspace), ws_bytes, N.stream_of(dev))
     return out
 
 

@@ -1,0 +1,101 @@
+"""GPU parity of the fp32 matrix-core decode kernel (head_dim 64 and 128, fp32 pools, page sizes
+other than 16, group sizes up to 16) against a 64-bit evaluation of the reference's decode
+(src/plastic_infer/exec/attention.py:151-190), at the edges of its 64 / 128-token tiles.
+
+Bars: scores, probabilities and sums are fp32, so a result is within 4e-6 of the row's largest
+|v| (128-term fp32 dot products of N(0, 1) data and a convex combination of v) before it is rounded
+once to the pool's dtype: one unit roundoff more for 16 bits (2^-8 / 2^-11 relative).
+"""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+from plastic_infer import _native as N
+from plastic_infer.kernel import paged_decode_append_attention, paged_decode_attention
+
+pytestmark = pytest.mark.gpu
+
+ROUNDOFF = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _reference(q, kp, vp, bt, lens, bad):
+    """64-bit decode; tokens on pages in `bad` (row, page index) are no keys."""
+    B, Hq, D = q.shape
+    P, Hkv = kp.shape[3], kp.shape[1]
+    out = torch.zeros(B, Hq, D, dtype=torch.float64)
+    for b, n in enumerate(lens.tolist()):
+        keep = [t for t in range(n) if (b, t // P) not in bad]
+        if not keep:
+            continue
+        t = torch.tensor(keep)
+        pg = bt[b].long()[t // P]
+        k, v = (x[pg, :, :, t % P].double() for x in (kp, vp))       # [n, Hkv, D]
+        qh = q[b].double().view(Hkv, Hq // Hkv, D)
+        p = torch.softmax(qh @ k.permute(1, 2, 0) / math.sqrt(D), -1)
+        out[b] = (p @ v.permute(1, 0, 2)).reshape(Hq, D)
+    return out
+
+
+@pytest.mark.parametrize("append", [False, True])
+@pytest.mark.parametrize("dtype,D,P,G", [
+    (torch.float32, 128, 16, 1), (torch.float32, 64, 4, 7), (torch.float32, 128, 12, 16),
+    (torch.bfloat16, 64, 16, 4), (torch.bfloat16, 128, 32, 4), (torch.float16, 64, 8, 3),
+    (torch.float16, 128, 16, 9), (torch.bfloat16, 128, 8, 16)])
+def test_decode_f32_tile_edges(dev, dtype, D, P, G, append):
+    Hkv, lens = 2, [1, 3, 63, 64, 65, 127, 128, 129, 0, 700, 2500, 255, 256, 257, 40, 130]
+    g = torch.Generator().manual_seed(D + P + G)
+    n_pages = [(n + P - 1) // P for n in lens]
+    total = sum(n_pages) + 3
+    perm = torch.randperm(total, generator=g)
+    bt = torch.full((len(lens), max(n_pages)), -1, dtype=torch.int32)
+    off = 0
+    for b, n in enumerate(n_pages):
+        bt[b, :n] = perm[off:off + n].to(torch.int32)
+        off += n
+    kp = torch.randn(total, Hkv, D, P, generator=g).to(dtype)
+    vp = torch.randn(total, Hkv, D, P, generator=g).to(dtype)
+    q = torch.randn(len(lens), Hkv * G + 2, D, generator=g).to(dtype)[:, :Hkv * G]
+    kn = torch.randn(len(lens), Hkv, D, generator=g).to(dtype)
+    vn = torch.randn(len(lens), Hkv, D, generator=g).to(dtype)
+    lens_t = torch.tensor(lens, dtype=torch.int32)
+    for b, n in enumerate(lens):                  # stale slots past the end hold NaN / Inf
+        if n % P:
+            kp[bt[b, n // P], :, :, n % P:] = float("nan")
+            vp[bt[b, n // P], :, :, n % P:] = float("inf")
+    bad = {(10, 3), (14, 0)} | {(14, i) for i in range(n_pages[14])}
+    bt_call = bt.clone()
+    for b, i in bad:                              # row 10 loses a page, row 14 all of them
+        bt_call[b, i] = total if i % 2 else -1
+    assert N.query("pia_paged_decode_split_scratch_bytes", Hkv * G, Hkv, D, P,
+                   N.dtype_code(dtype)) > 0
+    gk, gv = kp.to(dev), vp.to(dev)
+    args = (q.to(dev), gk, gv, bt_call.to(dev), lens_t.to(dev))
+    if append:
+        for b, n in enumerate(lens):
+            if n and (b, (n - 1) // P) not in bad:
+                kp[bt[b, (n - 1) // P], :, :, (n - 1) % P] = kn[b]
+                vp[bt[b, (n - 1) // P], :, :, (n - 1) % P] = vn[b]
+                gk[bt[b, (n - 1) // P], :, :, (n - 1) % P] = float("nan")
+                gv[bt[b, (n - 1) // P], :, :, (n - 1) % P] = float("inf")
+        out = paged_decode_append_attention(*args, kn.to(dev), vn.to(dev)).cpu()
+        for got, want in ((gk, kp), (gv, vp)):
+            assert torch.equal(got.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
+    else:
+        out = paged_decode_attention(*args).cpu()
+    ref = _reference(q, kp, vp, bt, lens_t, bad)
+    assert not out[8].any() and not out[14].any()
+    err = (out.double() - ref).abs()
+    assert (err <= ROUNDOFF[dtype] * 1.01 * ref.abs() + 4e-6 * 4.0).all(), err.max().item()
+    # the same call without scratch (general kernel) agrees within both kernels' error
+    if not append:
+        alone = torch.empty(q.shape, dtype=dtype, device=dev)
+        N.call("pia_paged_decode_attention", alone.data_ptr(), args[0].data_ptr(),
+               args[0].stride(0), gk.data_ptr(), gv.data_ptr(), args[3].data_ptr(), bt.shape[1],
+               args[4].data_ptr(), len(lens), Hkv * G, Hkv, D, P, total, 1.0 / math.sqrt(D),
+               N.dtype_code(dtype), None, 0, N.stream_of(dev))
+        diff = (alone.cpu().double() - out.double()).abs()
+        assert (diff <= 2.02 * ROUNDOFF[dtype] * ref.abs() + 2 * 4e-6 * 4.0).all()
