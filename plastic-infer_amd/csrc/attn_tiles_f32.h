@@ -128,23 +128,12 @@ __device__ __forceinline__ void qk(const uint4 (&kr)[16], const void* q,
   }
 }
 
-// 16-bit pair (pack16x2) back to fp32
-template <int DT>
-__device__ __forceinline__ float wide_lo(uint32_t x) {
-  if constexpr (DT == PIA_DTYPE_F16) return half_to_f32(uint16_t(x & 0xffffu));
-  else return bf16_lo(x);
-}
-template <int DT>
-__device__ __forceinline__ float wide_hi(uint32_t x) {
-  if constexpr (DT == PIA_DTYPE_F16) return half_to_f32(uint16_t(x >> 16));
-  else return bf16_hi(x);
-}
-
-// Eight fp32 values s[0..7][u] as three 16-bit operands whose sum they are: each term is what the
-// ones before leave, rounded to nearest. Three bf16 terms hold the 24 bits of any fp32 value that
-// is normal in all of them; three fp16 terms do for values of 2^-1 .. 2^15, below which the last
-// terms go denormal (the caller scales the probabilities by kSplitShift, so what is lost is under
-// 2^-39 of the largest).
+// Eight fp32 probabilities s[0..7][u] as three 16-bit operands whose sum they are, each term what
+// the ones before leave, rounded toward zero. Three bf16 terms hold the 24 bits of an fp32 value;
+// three fp16 terms do for values of 2^-1 .. 2^15 (the caller scales the probabilities by
+// kSplitShift, so what is lost is under 2^-39 of the largest). A positive value has three positive
+// terms (a zero one becomes the smallest denormal): times an infinite V they then give that
+// infinity, as the value itself would, and not infinity - infinity or 0 times infinity.
 template <int DT>
 constexpr float kSplitShift = DT == PIA_DTYPE_F16 ? 15.f : 0.f;  // log2 units
 template <int DT>
@@ -153,11 +142,26 @@ __device__ __forceinline__ void split3(const f32x4_t (&s)[8], int u, uint4 (&t)[
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
     float a = s[2 * f][u], b = s[2 * f + 1][u];
+    const uint32_t low =
+        min(__float_as_uint(a), 1u) | (min(__float_as_uint(b), 1u) << 16);  // 1 where positive
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      w[k][f] = tile::pack16x2<DT>(a, b);
-      a -= wide_lo<DT>(w[k][f]);
-      b -= wide_hi<DT>(w[k][f]);
+      if constexpr (DT == PIA_DTYPE_F16) {
+        const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
+        w[k][f] = __builtin_bit_cast(uint32_t, h);
+        a -= float(h[0]);
+        b -= float(h[1]);
+      } else {
+        w[k][f] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+        a -= bf16_hi(__float_as_uint(a));
+        b -= bf16_hi(__float_as_uint(b));
+      }
+      if (k > 0 || DT == PIA_DTYPE_F16) {  // a zero term of a positive value: the smallest one
+        typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+        w[k][f] = __builtin_bit_cast(
+            uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, w[k][f]),
+                                                __builtin_bit_cast(u16x2_t, low)));
+      }
     }
   }
 #pragma unroll

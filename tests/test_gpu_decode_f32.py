@@ -99,3 +99,19 @@ def test_decode_f32_tile_edges(dev, dtype, D, P, G, append):
                N.dtype_code(dtype), None, 0, N.stream_of(dev))
         diff = (alone.cpu().double() - out.double()).abs()
         assert (diff <= 2.02 * ROUNDOFF[dtype] * ref.abs() + 2 * 4e-6 * 4.0).all()
+
+
+@pytest.mark.parametrize("dtype", list(ROUNDOFF))
+def test_decode_f32_infinite_values(dev, dtype):
+    """V holds infinities: the result is that infinity (never infinity - infinity) for one key and
+    for many."""
+    q = torch.randn(2, 8, 64).to(dtype).to(dev)
+    kp, vp = (torch.randn(40, 2, 64, 16).to(dtype).to(dev) for _ in range(2))
+    vp[0, :, 5, 0] = float("-inf")
+    vp[3, :, 9, :8] = float("inf")
+    bt = torch.tensor([[0] + [1] * 19, [3] + list(range(4, 23))], dtype=torch.int32, device=dev)
+    out = paged_decode_attention(q, kp, vp, bt, torch.tensor([1, 300], dtype=torch.int32,
+                                                             device=dev)).cpu()
+    assert torch.equal(out[0].view(2, 4, 64), vp[0, :, :, 0].cpu().view(2, 1, 64).expand(-1, 4, -1))
+    assert (out[1, :, 9] == float("inf")).all()
+    assert out[1, :, torch.arange(64) != 9].isfinite().all()
