@@ -2742,6 +2742,11 @@ extern "C" int pia_paged_attention(void* out, const void* q, const void* k_pages
     return launch_prefill_mfma(dtype, out, q, k_pages, v_pages, block_tables, bt_stride, kv_lens,
                                cu_q, q_pos_offsets, num_seqs, total_q_rows, num_heads,
                                num_kv_heads, num_pages, scale * kLog2e, as_stream(stream));
+  if (rows_path(dtype, num_heads, num_kv_heads, head_dim, page_size, num_seqs, total_q_rows,
+                k_pages, v_pages))
+    return launch_rows(dtype, out, q, k_pages, v_pages, block_tables, bt_stride, kv_lens, cu_q,
+                       q_pos_offsets, num_seqs, total_q_rows, num_heads, num_kv_heads, head_dim,
+                       page_size, num_pages, scale * kLog2e, as_stream(stream));
   return launch_generic_any(dtype, out, q, int64_t(num_heads) * head_dim, k_pages, v_pages,
                             block_tables, bt_stride, kv_lens, cu_q, q_pos_offsets, num_seqs,
                             total_q_rows, num_heads, num_kv_heads, head_dim, page_size,

@@ -47,6 +47,16 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
                         int64_t total_q_rows, int Hq, int Hkv, int64_t num_pages,
                         float scale_log2, hipStream_t s);
 
+// Paged attention of any rows with fp32 precision on the matrix cores (paged_rows.hip): whether a
+// call takes it, and its launch (arguments already checked by pia_paged_attention).
+bool rows_path(int dtype, int Hq, int Hkv, int D, int P, int num_seqs, int64_t total_q_rows,
+               const void* k_pages, const void* v_pages);
+int launch_rows(int dtype, void* out, const void* q, const void* k_pages, const void* v_pages,
+                const int32_t* bt, int64_t bt_stride, const int32_t* kv_lens,
+                const int32_t* cu_q, const int32_t* offsets, int num_seqs, int64_t total_q_rows,
+                int Hq, int Hkv, int D, int P, int64_t num_pages, float scale_log2,
+                hipStream_t s);
+
 // ---------------------------------------------------------------------------------------------
 // Device helpers
 // ---------------------------------------------------------------------------------------------
