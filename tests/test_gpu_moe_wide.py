@@ -1,0 +1,103 @@
+"""GPU parity of the expert GEMM for many routes per expert (moe_gemm_wide) at the edges of its row
+tiles, K stages, column tiles and work lists, and of the one-launch permute plan, against the
+oracle. Bars as in test_gpu_fused_experts.py: fp32 sums in another order, then one rounding."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle.fused_experts as OF
+import oracle.moe_route as OM
+from plastic_infer.kernel import moe_align_block_size, moe_expert_gemm
+
+pytestmark = pytest.mark.gpu
+
+
+def _mostly_equal(got: torch.Tensor, ref: torch.Tensor, what: str):
+    got, ref = got.float().cpu(), ref.float().cpu()
+    diff = got != ref
+    assert diff.float().mean().item() < 0.01, what
+    if diff.any():
+        rel = ((got - ref).abs() / ref.abs().clamp_min(1e-2))[diff].max().item()
+        assert rel <= 4 * 2 ** -7, f"{what}: relative difference {rel}"
+
+
+def _ids(rows_of_expert, T, k, seed):
+    """Routes [T, k] that give expert e exactly rows_of_expert[e] of them, the rest -1."""
+    flat = np.concatenate([np.full(n, e) for e, n in enumerate(rows_of_expert)])
+    assert flat.size <= T * k
+    flat = np.concatenate([flat, np.full(T * k - flat.size, -1)])
+    return torch.tensor(np.random.default_rng(seed).permutation(flat).reshape(T, k),
+                        dtype=torch.int32)
+
+
+@pytest.mark.parametrize("rows,T,k,H,I,dtype,activation,on_input", [
+    # 64-row tiles (mean 18.75): none, one, 16 / 17 / 64 / 65 rows, an expert of four tiles
+    ([0, 1, 15, 16, 17, 63, 64, 65, 255] + [15] * 119, 300, 8, 328, 72, torch.bfloat16, "silu",
+     False),
+    # 128-row tiles (mean 80), K of whole stages and of one element vector more
+    ([127, 128, 129, 0, 300] + [60] * 27, 320, 8, 320, 200, torch.float16, "gelu", True),
+    # 192-row tiles (mean 150), short K: stages past its end
+    ([191, 192, 193, 385] + [80] * 12, 600, 4, 64, 136, torch.bfloat16, "gelu_tanh", False),
+    # 320-row tiles (mean 512): 319 / 320 / 321 rows and three tiles
+    ([319, 320, 321, 700, 1], 600, 4, 136, 264, torch.bfloat16, "silu", True),
+    # over 64 experts per XCD's work list
+    ([4] * 599 + [4], 300, 8, 72, 40, torch.float16, "silu", False),
+])
+def test_wide_expert_gemms(dev, rows, T, k, H, I, dtype, activation, on_input):
+    E, numel = len(rows), T * k
+    g = torch.Generator().manual_seed(E)
+    x = torch.randn(T, H, generator=g).to(dtype)
+    w1 = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(dtype)
+    w2 = (torch.randn(E, H, I, generator=g) * 0.05).to(dtype)
+    tw = torch.rand(T, k, generator=g)
+    ids = _ids(rows, T, k, E)
+    live = (ids >= 0).view(-1)
+    _, rc2, rc3 = OF.fused_experts(x, w1, w2, tw, ids.clamp_min(0), activation, on_input,
+                                   return_intermediate=True)
+    rc2, rc3 = torch.from_numpy(rc2).view(numel, I), torch.from_numpy(rc3).view(numel, H)
+    s, e, npp = moe_align_block_size(ids.to(dev), 16, E)
+    twd = tw.to(dev)
+    # a wider output row than its columns, and rows of dropped routes left alone
+    out = torch.full((numel, I + 3), 7.0, dtype=dtype, device=dev)
+    c2 = moe_expert_gemm(x.to(dev), w1.to(dev), twd, s, e, npp, 16, numel, k,
+                         activation=activation, mul_routed_weight=on_input, out=out[:, :I])
+    _mostly_equal(c2.cpu()[live], rc2[live], "first GEMM + activation")
+    assert bool((out.cpu()[~live] == 7.0).all()) and bool((out[:, I:] == 7.0).all())
+    c3 = moe_expert_gemm(rc2.to(dtype).to(dev), w2.to(dev), twd, s, e, npp, 16, numel, 1,
+                         mul_routed_weight=not on_input)
+    _mostly_equal(c3.cpu()[live], rc3[live], "second GEMM")
+
+
+@pytest.mark.parametrize("n_rows,K", [(100, 328), (250, 64), (257, 640)])
+def test_wide_odd_columns(dev, n_rows, K):
+    """Output columns that are no multiple of a store's eight."""
+    T, k, E = 520, 4, 8
+    g = torch.Generator().manual_seed(n_rows)
+    a = torch.randn(T * k, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(E, n_rows, K, generator=g) * 0.05).to(torch.bfloat16)
+    ids = torch.randint(0, E, (T, k), generator=g).to(torch.int32)
+    s, e, npp = moe_align_block_size(ids.to(dev), 16, E)
+    got = moe_expert_gemm(a.to(dev), w.to(dev), None, s, e, npp, 16, T * k, 1)
+    ref = torch.stack([w[x].float() @ r for x, r in zip(ids.view(-1).tolist(), a.float())])
+    _mostly_equal(got, ref.to(torch.bfloat16), "odd columns")
+
+
+@pytest.mark.parametrize("T,k,E,skew", [(1, 1, 1, 0), (128, 8, 2, 0), (512, 8, 255, 1),
+                                        (129, 8, 2047, 0), (512, 8, 2048, 0), (205, 5, 300, 1)])
+def test_one_launch_plan(dev, T, k, E, skew):
+    """The plan of up to 4096 routes: rounds of 1024, waves that share an expert, and either side
+    of the largest expert count that has per-wave counters."""
+    rng = np.random.default_rng(T + E)
+    ids = rng.integers(-1, E + 2, size=(T, k)).astype(np.int32)
+    if skew:                                    # most routes to one expert
+        ids[rng.random((T, k)) < 0.8] = E - 1
+    rs, re, rnpp, rpos = OM.moe_align_block_size(ids, 16, E)
+    s, e, npp, pos = moe_align_block_size(torch.tensor(ids, device=dev), 16, E,
+                                          return_route_pos=True)
+    assert int(npp.item()) == rnpp
+    assert np.array_equal(s.cpu().numpy(), rs)
+    assert np.array_equal(e.cpu().numpy()[:rnpp // 16], re[:rnpp // 16])
+    assert np.array_equal(pos.cpu().numpy(), rpos)
