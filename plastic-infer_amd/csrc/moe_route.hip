@@ -684,7 +684,7 @@ __global__ __launch_bounds__(1024) void moe_align_small(
   // wave's routes of its expert comes from one ballot per bit of the expert index; each wave's
   // counts meet in LDS (a byte per expert and wave: an expert's sixteen in one 16-byte read), and
   // a lane adds those of the waves before its own. Two barriers per round; the waves in turn took 17.4 us for 2664 routes of 128 experts and
-  // 6.3 us for 16 (this: 7.0 and 5.3).
+  // 6.3 us for 16 (this: 8.0 and 4.4).
   const int bits = 32 - __builtin_clz(E_eff);
   for (int g0 = 0; g0 < numel; g0 += 1024) {
     const int i = g0 + tid;
