@@ -347,6 +347,22 @@ int pia_moe_unpermute(void* out, const void* y, int64_t y_rows, const int32_t* r
 int pia_moe_sum_reduce(void* out, const void* in, int64_t num_tokens, int topk, int hidden_dim,
                        int dtype, void* stream);
 
+/* out = s / sqrt(mean(s^2) + eps) * weight over rows of n elements, s = x, or x + residual rounded
+ * to the dtype and written to sum (a buffer of its own) when residual is given. The
+ * reference's rms_norm (src/plastic_infer/exec/attention.py:77-79) with fp32 arithmetic and one
+ * rounding. */
+int pia_rms_norm(void* out, void* sum, const void* x, const void* residual, const void* weight,
+                 int64_t rows, int n, float eps, int dtype, void* stream);
+
+/* Per-head RMSNorm (both weights NULL: none), then rotate-half RoPE: q [rows, num_heads, head_dim]
+ * and k [rows, num_kv_heads, head_dim] by the rows' table rows cos, sin [rows, head_dim]; fp32
+ * arithmetic, one rounding (reference: qk_norm and RoPE,
+ * src/plastic_infer/exec/attention.py:53-95). */
+int pia_qk_norm_rope(void* q_out, void* k_out, const void* q, const void* k, const void* q_weight,
+                     const void* k_weight, const void* cos, const void* sin, int64_t rows,
+                     int num_heads, int num_kv_heads, int head_dim, float eps, int dtype,
+                     void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Grouped expert GEMM over a permute plan, one of the two GEMMs of the fused experts FFN
  * (fused_experts_impl / fused_experts_decode_impl, reference src/plastic_infer/moe/fused.py:

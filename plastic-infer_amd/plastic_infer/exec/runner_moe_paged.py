@@ -11,10 +11,10 @@ at once. Every layer of a step does, for all B rows:
   RMSNorm -> router logits -> softmax top-k with renormalised weights -> routed expert FFN
   over the slot cache -> residual;
 
-then the final RMSNorm and the LM head give [B, vocab] logits. The projections, norms and RoPE
-are plain torch ops in the model dtype with the reference's formulas (RoPE tables built in the
-model dtype, as the reference builds them); the KV, attention, routing and expert data path is
-this package's HIP kernels.
+then the final RMSNorm and the LM head give [B, vocab] logits. The projections are plain torch
+ops in the model dtype; the norms (with the residual add before them) and RoPE are one launch each
+with the reference's formulas (RoPE tables built in the model dtype, as the reference builds them),
+and the KV, attention, routing and expert data path is this package's HIP kernels.
 
 Routed experts, overlapped (overlap=True): the cache plans the layer's misses on the host and
 copies them with the DMA engines on its copy stream (OffloadMoeCache.stage_layer); the FFN of
@@ -37,11 +37,12 @@ import torch
 import torch.nn.functional as F
 
 from ..kernel.moe_ops import moe_sum_reduce
+from ..kernel.norm_rope import add_rms_norm_rows, qk_norm_rope, rms_norm_rows
 from ..kernel.paged_kv import decode_workspace_bytes, paged_decode_append_attention
 from ..kernel.pinned import alloc_pinned_exact
 from ..moe.fused import fused_experts_decode_impl, fused_topk, routed_ffn_routes
 from ..moe.offload_cache import OffloadMoeCache
-from .attention import build_rope_cache, rms_norm
+from .attention import build_rope_cache
 
 
 @dataclass
@@ -176,13 +177,6 @@ class MoePagedDecoder:
 
     # ---- pieces --------------------------------------------------------------------------------
 
-    def _rope(self, x: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
-        """RoPE of x [B, heads, D], row b at position pos[b] (rotate-half form)."""
-        c = self.cos[pos][:, None, :]
-        s = self.sin[pos][:, None, :]
-        x1, x2 = x.chunk(2, dim=-1)
-        return x * c + torch.cat([-x2, x1], dim=-1) * s
-
     def _routed(self, layer: int, h: torch.Tensor, topk_w: torch.Tensor,
                 topk_ids: torch.Tensor) -> tuple[torch.Tensor, dict]:
         gate_up, down = self.cache.bank_views()
@@ -205,50 +199,63 @@ class MoePagedDecoder:
             ev["a1"] = torch.cuda.Event(enable_timing=True)
             ev["a1"].record(compute)
         compute.wait_event(routes.ready)
-        routed_ffn_routes(h, gate_up, down, topk_w, routes.copied, route_out, act_buffer=act)
+        if routes.copied_experts:   # else every route was in the first group
+            routed_ffn_routes(h, gate_up, down, topk_w, routes.copied, route_out, act_buffer=act)
         out = torch.empty_like(h)
         moe_sum_reduce(route_out, out)
-        return out, {"routes": routes, "events": ev,
-                     "slots": torch.maximum(routes.in_hbm, routes.copied)}
+        info = {"routes": routes, "events": ev}
+        if self.layer_hook is not None:
+            info["slots"] = torch.maximum(routes.in_hbm, routes.copied)
+        return out, info
 
     # ---- one step ------------------------------------------------------------------------------
 
     def step(self, input_ids: torch.Tensor, batch: DecodeBatch) -> torch.Tensor:
         """One decode token for every row: [B] token ids -> [B, vocab] logits."""
         cfg, w = self.cfg, self.w
-        B = input_ids.shape[0]
-        Hq, Hkv, D = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
         x = w["embed_tokens.weight"][input_ids].to(cfg.dtype)
+        rope = self._rope_rows(batch)
+        norms = [w[f"layers.{l}.input_layernorm.weight"] for l in range(cfg.n_layers)]
+        norms.append(w["norm.weight"])
+        h = rms_norm_rows(x, norms[0])
         for l in range(cfg.n_layers):
-            x = self.layer(l, x, batch)
-        x = rms_norm(x, w["norm.weight"])
-        return F.linear(x, w["lm_head.weight"])
+            x, routed = self._layer(l, x, h, batch, rope)
+            x, h = add_rms_norm_rows(x, routed, norms[l + 1])
+        return F.linear(h, w["lm_head.weight"])
 
     def layer(self, l: int, x: torch.Tensor, batch: DecodeBatch) -> torch.Tensor:
         """One decoder layer for all rows: x [B, hidden] -> [B, hidden]."""
+        h = rms_norm_rows(x, self.w[f"layers.{l}.input_layernorm.weight"])
+        x, routed = self._layer(l, x, h, batch, self._rope_rows(batch))
+        return x + routed
+
+    def _rope_rows(self, batch: DecodeBatch) -> tuple[torch.Tensor, torch.Tensor]:
+        """The rows' cos / sin table rows [B, D]: every layer of a step takes the same."""
+        return self.cos[batch.positions], self.sin[batch.positions]
+
+    def _layer(self, l: int, x: torch.Tensor, h: torch.Tensor, batch: DecodeBatch,
+               rope: tuple[torch.Tensor, torch.Tensor]) -> tuple[torch.Tensor, torch.Tensor]:
+        """A layer from its input x and that input's norm h: (x after attention, the routed
+        experts' output), whose sum is the layer's output."""
         cfg, w = self.cfg, self.w
         B = x.shape[0]
         Hq, Hkv, D = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
         p = f"layers.{l}."
-        residual = x
-        h = rms_norm(x, w[p + "input_layernorm.weight"])
         q = F.linear(h, w[p + "self_attn.q_proj.weight"]).view(B, Hq, D)
         k = F.linear(h, w[p + "self_attn.k_proj.weight"]).view(B, Hkv, D)
         v = F.linear(h, w[p + "self_attn.v_proj.weight"]).view(B, Hkv, D)
-        if cfg.qk_norm:
-            q = rms_norm(q, w[p + "self_attn.q_norm.weight"])
-            k = rms_norm(k, w[p + "self_attn.k_norm.weight"])
-        q = self._rope(q, batch.positions).contiguous()
-        k = self._rope(k, batch.positions).contiguous()
+        qk_weights = (w[p + "self_attn.q_norm.weight"], w[p + "self_attn.k_norm.weight"]) \
+            if cfg.qk_norm else (None, None)
+        q, k = qk_norm_rope(q, k, *qk_weights, *rope)
         v = v.contiguous()
         # the reference's _write_kv_layer then _attn_paged, as one call: the new token goes to
         # its slot and the attention takes it from k / v directly
         attn = paged_decode_append_attention(q, self.k_pages, self.v_pages,
                                              batch.block_tables[l], batch.context_lens, k, v,
                                              workspace=self._ws)
-        x = residual + F.linear(attn.view(B, Hq * D), w[p + "self_attn.o_proj.weight"])
-        residual = x
-        h = rms_norm(x, w[p + "post_attention_layernorm.weight"])
+        x, h = add_rms_norm_rows(x, F.linear(attn.view(B, Hq * D),
+                                             w[p + "self_attn.o_proj.weight"]),
+                                 w[p + "post_attention_layernorm.weight"])
         logits = F.linear(h, w[p + "mlp.router.weight"])
         topk_w, topk_ids = fused_topk(h, logits, cfg.n_experts_per_tok, True)
         routed, info = self._routed(l, h, topk_w, topk_ids)
@@ -256,7 +263,7 @@ class MoePagedDecoder:
             self.layer_hook(l, {"q": q, "k": k, "v": v, "attn": attn, "moe_in": h,
                                 "topk_weights": topk_w, "topk_ids": topk_ids, "routed": routed,
                                 **info})
-        return residual + routed
+        return x, routed
 
 
 __all__ = ["MoeModelConfig", "qwen3_30b_a3b_config", "random_dense_weights",
