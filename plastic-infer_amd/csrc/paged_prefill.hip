@@ -41,11 +41,10 @@
 // Keys a row may not see (past its causal limit or the sequence's length, on a page whose
 // block-table id is outside the pool) score -inf; their V words are zeros from the loads.
 //
-// Work list: sequence-major, then kv head, then position tile (the last tiles of a sequence,
-// which see the most keys when causal, first). A 1-D grid is dispatched round-robin over the 8
-// XCDs (workgroup i runs on XCD i % 8); the list is cut into 8 contiguous runs and XCD x takes
-// run x in order, so the ~64 workgroups resident on one XCD are the position tiles of one
-// (sequence, kv head) and read its K / V through that XCD's L2 once between them.
+// Work list: by kv head, sequence, position tile (the last tiles of a sequence, which see the most
+// keys when causal, first), with the heads dealt to the XCDs (xcd_item), so the ~64 workgroups
+// resident on one XCD are the position tiles of one (sequence, kv head) or a few and read its
+// K / V through that XCD's L2 once between them.
 #include <algorithm>
 
 #include "attn_tiles.h"
@@ -81,7 +80,6 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_mfma(
   constexpr int NT = 64 * NW;                 // threads per workgroup
   constexpr int PPT = PF_WROWS * NW / G;  // query positions per work item
   constexpr int RB = PF_RB;
-  constexpr int XCDS = 8;
   __shared__ __align__(16) uint16_t ks[2][PF_D * PF_KT];
   __shared__ __align__(16) uint16_t vs[2][PF_D * PF_KT];
   __shared__ int tile_pref[PF_MAX_SEQS + 1];
@@ -112,22 +110,16 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_mfma(
     for (int x = 0; x < NW; ++x) carry += wsum[x];
     __syncthreads();
   }
-  // this workgroup's item: XCD x = blockIdx % 8 runs items [x * run, (x + 1) * run) in order
-  const int64_t items = int64_t(carry) * Hkv;
-  const int64_t run = (items + XCDS - 1) / XCDS;
-  const int64_t k = blockIdx.x / XCDS;
-  const int64_t item = (blockIdx.x % XCDS) * run + k;
-  if (k >= run || item >= items) return;
-  int lo = 0, hi = B - 1;  // the sequence holding the item: Hkv * tile_pref[b] <= item
+  // this workgroup's item: its kv head, and item j of that head over the sequences in order
+  int h, j;
+  if (!xcd_item(blockIdx.x, carry, Hkv, h, j)) return;
+  int lo = 0, hi = B - 1;  // the sequence holding the item: the last with tile_pref[b] <= j
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (int64_t(tile_pref[mid]) * Hkv <= item) lo = mid; else hi = mid - 1;
+    if (tile_pref[mid] <= j) lo = mid; else hi = mid - 1;
   }
   const int b = lo;
-  const int nt_b = tile_pref[b + 1] - tile_pref[b];
-  const int rem = int(item - int64_t(tile_pref[b]) * Hkv);
-  const int h = rem / nt_b;
-  const int s0 = (nt_b - 1 - rem % nt_b) * PPT;
+  const int s0 = (tile_pref[b + 1] - 1 - j) * PPT;
   const int64_t row0 = cu_q ? int64_t(cu_q[b]) : int64_t(b);
   const int n_b = cu_q ? cu_q[b + 1] - cu_q[b] : 1;
   int kv_len = kv_lens[b];
@@ -457,8 +449,12 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
                         float scale_log2, hipStream_t s) {
   const int G = Hq / Hkv;
   // eight waves (256 rows per item, one K / V tile staged for all of them) when the sequences
-  // average at least half an item, else four (128 rows)
-  const bool wide = 2 * total_q_rows >= int64_t(8 * PF_WROWS / G) * num_seqs;
+  // average at least half an item and the items fill the compute units twice over, else four
+  // (128 rows): 312 items of 8 sequences of 100..800 rows, 16/8 heads, 75.8 us against 64.9 with
+  // four; 72 items of one sequence of 300 rows behind 1500 tokens, 32/8 heads, 63.5 against 55.2
+  const int wide_ppt = 8 * PF_WROWS / G;
+  const bool wide = 2 * total_q_rows >= int64_t(wide_ppt) * num_seqs &&
+                    (ceil_div(total_q_rows, wide_ppt) + num_seqs) * Hkv >= 2 * int64_t(device_cus());
   const int ppt = (wide ? 8 : 4) * PF_WROWS / G;
   // work items: at most ceil(total rows / ppt) + one partial item per sequence
   const int64_t items = (ceil_div(total_q_rows, ppt) + num_seqs) * Hkv;

@@ -12,8 +12,8 @@
 // over the waves, not the rows, keeps short prompts' few row blocks on four times the SIMDs and
 // needs no barrier in the loop. fp32 pools are bound by the 16x16x4 products (32 cycles for 2048
 // FLOP); 16-bit pools by the tile reads from L2: 64 KiB (D = 128) for each 16 rows and tile.
-// Work list order and XCD runs as in paged_prefill_mfma: the items of one (sequence, kv head)
-// run on one XCD, whose L2 holds its K / V.
+// Work list as in paged_prefill_mfma: the items of one (sequence, kv head) run on one XCD or few,
+// whose L2 holds its K / V.
 //
 // A row sees keys below its own limit; the other keys of a tile score -inf. Tokens that no row of
 // the item sees have their V components zeroed. A token that only some of the rows see may hold a
@@ -22,7 +22,7 @@
 //
 // Measured against paged_attention_tiled, which ran a workgroup per row: 2 sequences of 300..600
 // rows behind 0..512 tokens, 16/8 heads of 128, fp32:
-// 743 -> 116 us.
+// 743 -> 116 us, and 98 us with the heads dealt to the XCDs.
 #include <algorithm>
 
 #include "attn_tiles.h"
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
   constexpr int TV = V::TV, TOK = V::TOKENS, NB = D / 16, NI = D / 4;
   constexpr int NU = D == 128 ? 2 : 4;          // V vectors u of one register buffer
   constexpr int QS = NI + 16 / int(sizeof(T));  // LDS stride of a lane's q elements
-  constexpr int NT = 64 * PR_WAVES, XCDS = 8;
+  constexpr int NT = 64 * PR_WAVES;
   __shared__ int item_pref[PR_MAX_SEQS + 1];
   __shared__ int wsum[PR_WAVES];
   __shared__ __align__(16) T qs[64 * QS];  // [lane]: q[row n16][4 i + kd] (fp32: pre-scaled)
@@ -97,22 +97,16 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
     for (int x = 0; x < PR_WAVES; ++x) carry += wsum[x];
     __syncthreads();
   }
-  // this workgroup's item: XCD x = blockIdx % 8 runs items [x * run, (x + 1) * run) in order
-  const int64_t items = int64_t(carry) * Hkv;
-  const int64_t run = (items + XCDS - 1) / XCDS;
-  const int64_t slot = blockIdx.x / XCDS;
-  const int64_t item = (blockIdx.x % XCDS) * run + slot;
-  if (slot >= run || item >= items) return;
-  int lo = 0, hi = B - 1;  // the sequence holding the item: Hkv * item_pref[b] <= item
+  // this workgroup's item: its kv head, and item j of that head over the sequences in order
+  int h, j;
+  if (!xcd_item(blockIdx.x, carry, Hkv, h, j)) return;
+  int lo = 0, hi = B - 1;  // the sequence holding the item: the last with item_pref[b] <= j
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (int64_t(item_pref[mid]) * Hkv <= item) lo = mid; else hi = mid - 1;
+    if (item_pref[mid] <= j) lo = mid; else hi = mid - 1;
   }
   const int b = lo;
-  const int n_it = item_pref[b + 1] - item_pref[b];
-  const int rem = int(item - int64_t(item_pref[b]) * Hkv);
-  const int h = rem / n_it;
-  const int R0 = (n_it - 1 - rem % n_it) * PR_ROWS;  // the last rows, with the most keys, first
+  const int R0 = (item_pref[b + 1] - 1 - j) * PR_ROWS;  // the last rows, with the most keys, first
   const int64_t row0 = cu_q ? int64_t(cu_q[b]) : int64_t(b);
   const int n_rows = rows_of(b) * G;  // flat rows of the (sequence, kv head)
   int kv_len = kv_lens[b];

@@ -61,6 +61,24 @@ int launch_rows(int dtype, void* out, const void* q, const void* k_pages, const 
 // Device helpers
 // ---------------------------------------------------------------------------------------------
 
+// Work list of the multi-row attention kernels: workgroup `block` (on XCD block % 8) of a call with
+// n items per kv head takes item `j` of kv head `h`; false: none. An XCD runs whole heads where
+// 8 divides their number, else it shares heads with others, item by item, so that every XCD gets
+// the same part of every sequence: K / V of a (sequence, head) go through one XCD's L2 (or few),
+// and sequences of different lengths do not load the XCDs differently, as contiguous runs of a
+// sequence-major list did (2 sequences, 16/8 heads, fp32: 1.2 of 2 waves per SIMD in flight).
+__device__ __forceinline__ bool xcd_item(int64_t block, int n, int Hkv, int& h, int& j) {
+  const int own = Hkv % 8 == 0 ? 8 : Hkv % 4 == 0 ? 4 : Hkv % 2 == 0 ? 2 : 1;  // head classes
+  const int share = 8 / own;                                                   // XCDs of a class
+  const int x = int(block % 8);
+  const int64_t l = (block / 8) * share + x / own;
+  if (l >= int64_t(Hkv / own) * n) return false;
+  const int i = int(l / n);
+  h = x % own + own * i;
+  j = int(l - int64_t(i) * n);
+  return true;
+}
+
 // bf16 <-> f32 by bit manipulation (bf16 is the upper half of an IEEE binary32).
 __device__ __forceinline__ float bf16_lo(uint32_t x) { return __uint_as_float(x << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t x) { return __uint_as_float(x & 0xffff0000u); }
