@@ -41,6 +41,9 @@
 // Keys a row may not see (past its causal limit or the sequence's length, on a page whose
 // block-table id is outside the pool) score -inf; their V words are zeros from the loads.
 //
+// Few items with many keys: two groups of four waves take every other tile of an item's keys, each
+// with its own buffers, maxima and sums, and meet in LDS at the end (template parameter KS).
+//
 // Work list: by kv head, sequence, position tile (the last tiles of a sequence, which see the most
 // keys when causal, first), with the heads dealt to the XCDs (xcd_item), so the ~64 workgroups
 // resident on one XCD are the position tiles of one (sequence, kv head) or a few and read its
@@ -69,30 +72,30 @@ constexpr int PF_RSRC_WORD3 = 0x00020000;
 // that trails its true max by at most this much, so probabilities stay <= 2^8
 constexpr float PF_RESCALE = 8.0f;
 
-template <int G, int NW, int DT>
-__global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_mfma(
+template <int G, int NW, int KS, int DT>
+__global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfma(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ q,
     const uint16_t* __restrict__ kpool, const uint16_t* __restrict__ vpool,
     const int32_t* __restrict__ bt, int64_t bt_stride, const int32_t* __restrict__ kv_lens,
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ offsets, int B, int Hkv,
     int64_t num_pages, float scale_log2) {
   constexpr int D = PF_D, P = PF_P, TILE = D * P;
-  constexpr int NT = 64 * NW;                 // threads per workgroup
+  constexpr int NT = 64 * NW * KS;        // threads per workgroup
   constexpr int PPT = PF_WROWS * NW / G;  // query positions per work item
   constexpr int RB = PF_RB;
-  __shared__ __align__(16) uint16_t ks[2][PF_D * PF_KT];
-  __shared__ __align__(16) uint16_t vs[2][PF_D * PF_KT];
+  __shared__ __align__(16) uint16_t ks_all[KS][2][PF_D * PF_KT];
+  __shared__ __align__(16) uint16_t vs_all[KS][2][PF_D * PF_KT];
   __shared__ int tile_pref[PF_MAX_SEQS + 1];
-  __shared__ int wsum[NW];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ int wsum[NW * KS];
+  const int lane = threadIdx.x & 63;
   const int Hq = Hkv * G;
   const int64_t q_row = int64_t(Hq) * D;  // elements between query positions
 
   // work items per sequence (ceil(rows / PPT)) and their prefix, scanned NT sequences at a time
-  if (tid == 0) tile_pref[0] = 0;
+  if (threadIdx.x == 0) tile_pref[0] = 0;
   int carry = 0;
   for (int c0 = 0; c0 < B; c0 += NT) {
-    const int i = c0 + tid;
+    const int i = c0 + threadIdx.x, wave_all = threadIdx.x >> 6;
     const int n = i < B ? (cu_q ? cu_q[i + 1] - cu_q[i] : 1) : 0;
     const int t = n > 0 ? (n + PPT - 1) / PPT : 0;
     int incl = t;
@@ -101,13 +104,13 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_mfma(
       const int y = __shfl_up(incl, o, 64);
       if (lane >= o) incl += y;
     }
-    if (lane == 63) wsum[wave] = incl;
+    if (lane == 63) wsum[wave_all] = incl;
     __syncthreads();
     int base = carry;
-    for (int x = 0; x < wave; ++x) base += wsum[x];
+    for (int x = 0; x < wave_all; ++x) base += wsum[x];
     if (i < B) tile_pref[i + 1] = base + incl;
 #pragma unroll
-    for (int x = 0; x < NW; ++x) carry += wsum[x];
+    for (int x = 0; x < NW * KS; ++x) carry += wsum[x];
     __syncthreads();
   }
   // this workgroup's item: its kv head, and item j of that head over the sequences in order
@@ -131,6 +134,12 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_mfma(
   const int npages = (kv_len + P - 1) / P;
   const int nkt = (kmax + PF_KT - 1) / PF_KT;
   const int32_t* btb = bt + int64_t(b) * bt_stride;
+
+  // key group (which of every KS tiles), and thread and wave inside it
+  const int kgrp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / (64 * NW));
+  const int tid = threadIdx.x - kgrp * 64 * NW, wave = tid >> 6;
+  uint16_t(*ks)[PF_D * PF_KT] = ks_all[kgrp];
+  uint16_t(*vs)[PF_D * PF_KT] = vs_all[kgrp];
 
   // this lane's score rows: 32 wave + 16 rb + l % 16 (rb < RB) and their q operands,
   // d = 32 kc + 8 (l / 16) .. + 7
@@ -283,133 +292,176 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void paged_prefill_mfma(
   // the buffer the tile read. The fetches run unconditionally (past the last tile they load
   // data no stage uses): with no branch around them, the wait for the block-table load issued
   // before a fetch counts exactly the fetch's loads instead of waiting for all of them.
-  int bt_cur = bt_of(0), bt_nxt = bt_of(1), bt_far = bt_of(2);
+  int bt_cur = bt_of(kgrp), bt_nxt = bt_of(kgrp + KS), bt_far = bt_of(kgrp + 2 * KS);
   fetch(bt_cur);
-  stage(0, 0);
+  stage(0, kgrp);
   fetch(bt_nxt);
   __syncthreads();
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int buf = kt & 1;
+  for (int it = 0; it * KS < nkt; ++it) {
+    const int kt = it * KS + kgrp, buf = it & 1;
+    const bool real = KS == 1 || kt < nkt;  // a group past its last tile only keeps the barriers
     const int pmask = page_mask(bt_cur);
     // a tile every valid row sees whole (interior of the causal triangle, all pages valid)
     const bool full = pmask == 0xF && (kt + 1) * PF_KT <= lim_min;
-    const int bt_next_far = bt_of(kt + 3);
+    const int bt_next_far = bt_of(kt + 3 * KS);
 
     // S^T for the wave's rows: 4 token blocks (one per page) x 4 d chunks, each K operand
     // serving both row blocks; d chunk outermost, so consecutive products of one accumulator
     // are 4 RB MFMAs apart (a product that reads the result of the one just issued waits for
     // it to drain)
-    f32x4_t sc[RB][4];
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const uint2 lo = tile::read_tr16(&ks[buf][(k_base[0] ^ (16 * mb)) + 2048 * kc]);
-        const uint2 hi = tile::read_tr16(&ks[buf][(k_base[1] ^ (16 * mb)) + 2048 * kc]);
-        const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-          sc[rb][mb] = tile::mfma16<DT>(a, qreg[rb][kc],
-                                       kc == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : sc[rb][mb]);
-      }
-    }
     uint4 pk[RB][2];
-    bool moved = false;
-    float alpha[RB];
+    if (real) {
+      f32x4_t sc[RB][4];
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      // on boundary tiles, keys the row may not see (tokens 64 kt + 16 mb + 4 g4 + j) -> -inf
-      if (!full) {
-        // token 64 kt + 16 mb + 4 g4 + j is visible to the row when 16 mb + j < rel (one
-        // per-lane value and immediates: written with the token index per element, the
-        // compiler computed all sixteen indices ahead of the branch, on every tile)
-        const int rel = lim_r[rb] - (kt * PF_KT + 4 * g4);
+      for (int kc = 0; kc < 4; ++kc) {
 #pragma unroll
-        for (int mb = 0; mb < 4; ++mb)
+        for (int mb = 0; mb < 4; ++mb) {
+          const uint2 lo = tile::read_tr16(&ks[buf][(k_base[0] ^ (16 * mb)) + 2048 * kc]);
+          const uint2 hi = tile::read_tr16(&ks[buf][(k_base[1] ^ (16 * mb)) + 2048 * kc]);
+          const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (!(16 * mb + j < rel && ((pmask >> mb) & 1))) sc[rb][mb][j] = -INFINITY;
+          for (int rb = 0; rb < RB; ++rb)
+            sc[rb][mb] = tile::mfma16<DT>(a, qreg[rb][kc],
+                                         kc == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : sc[rb][mb]);
+        }
       }
-      // the row max with IEEE 754-2019 maximum (a NaN score makes it NaN, and the row's output
-      // NaN, as the reference's softmax gives): v_maximum3_f32, no quieting of the scores
-      float mx = -INFINITY;
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-        mx = __builtin_elementwise_maximum(
-            mx, __builtin_elementwise_maximum(
-                    __builtin_elementwise_maximum(sc[rb][mb][0], sc[rb][mb][1]),
-                    __builtin_elementwise_maximum(sc[rb][mb][2], sc[rb][mb][3])));
-      mx = tile::maximum_col4(mx);
-      // move the reference point only for a large enough rise (or the first keys of the row)
-      const float mref = (mx - m[rb]) * scale_log2 > PF_RESCALE ? mx : m[rb];
-      alpha[rb] = m[rb] == mref ? 1.f : __builtin_amdgcn_exp2f((m[rb] - mref) * scale_log2);
-      moved = moved || m[rb] != mref;
-      m[rb] = mref;
-      // p = 2^((s - m) * scale_log2); a row with no key yet keeps m = -inf and p = 0
-      const float nm = mref == -INFINITY ? 0.f : -mref * scale_log2;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        float p[2][4];
-#pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            p[hh][j] = __builtin_amdgcn_exp2f(fmaf(sc[rb][2 * c + hh][j], scale_log2, nm));
-        pk[rb][c] = make_uint4(
-            tile::pack16x2<DT>(p[0][0], p[0][1]), tile::pack16x2<DT>(p[0][2], p[0][3]),
-            tile::pack16x2<DT>(p[1][0], p[1][1]), tile::pack16x2<DT>(p[1][2], p[1][3]));
-      }
-    }
-    // rescale O and the sums when some row's reference point moved: lane l's accumulator rows
-    // are 4 g4 + j of each block; their alpha sits in lane 4 g4 + j
-    if (__ballot(moved)) {
+      bool moved = false;
+      float alpha[RB];
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
-        float aj[4];
+        // on boundary tiles, keys the row may not see (tokens 64 kt + 16 mb + 4 g4 + j) -> -inf
+        if (!full) {
+          // token 64 kt + 16 mb + 4 g4 + j is visible to the row when 16 mb + j < rel (one
+          // per-lane value and immediates: written with the token index per element, the
+          // compiler computed all sixteen indices ahead of the branch, on every tile)
+          const int rel = lim_r[rb] - (kt * PF_KT + 4 * g4);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) aj[j] = __shfl(alpha[rb], 4 * g4 + j, 64);
+          for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          lsum[rb][j] *= aj[j];
+            for (int j = 0; j < 4; ++j)
+              if (!(16 * mb + j < rel && ((pmask >> mb) & 1))) sc[rb][mb][j] = -INFINITY;
+        }
+        // the row max with IEEE 754-2019 maximum (a NaN score makes it NaN, and the row's output
+        // NaN, as the reference's softmax gives): v_maximum3_f32, no quieting of the scores
+        float mx = -INFINITY;
 #pragma unroll
-          for (int nb = 0; nb < 8; ++nb) acc[rb][nb][j] *= aj[j];
+        for (int mb = 0; mb < 4; ++mb)
+          mx = __builtin_elementwise_maximum(
+              mx, __builtin_elementwise_maximum(
+                      __builtin_elementwise_maximum(sc[rb][mb][0], sc[rb][mb][1]),
+                      __builtin_elementwise_maximum(sc[rb][mb][2], sc[rb][mb][3])));
+        mx = tile::maximum_col4(mx);
+        // move the reference point only for a large enough rise (or the first keys of the row)
+        const float mref = (mx - m[rb]) * scale_log2 > PF_RESCALE ? mx : m[rb];
+        alpha[rb] = m[rb] == mref ? 1.f : __builtin_amdgcn_exp2f((m[rb] - mref) * scale_log2);
+        moved = moved || m[rb] != mref;
+        m[rb] = mref;
+        // p = 2^((s - m) * scale_log2); a row with no key yet keeps m = -inf and p = 0
+        const float nm = mref == -INFINITY ? 0.f : -mref * scale_log2;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          float p[2][4];
+#pragma unroll
+          for (int hh = 0; hh < 2; ++hh)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              p[hh][j] = __builtin_amdgcn_exp2f(fmaf(sc[rb][2 * c + hh][j], scale_log2, nm));
+          pk[rb][c] = make_uint4(
+              tile::pack16x2<DT>(p[0][0], p[0][1]), tile::pack16x2<DT>(p[0][2], p[0][3]),
+              tile::pack16x2<DT>(p[1][0], p[1][1]), tile::pack16x2<DT>(p[1][2], p[1][3]));
+        }
+      }
+      // rescale O and the sums when some row's reference point moved: lane l's accumulator rows
+      // are 4 g4 + j of each block; their alpha sits in lane 4 g4 + j
+      if (__ballot(moved)) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+          float aj[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) aj[j] = __shfl(alpha[rb], 4 * g4 + j, 64);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            lsum[rb][j] *= aj[j];
+#pragma unroll
+            for (int nb = 0; nb < 8; ++nb) acc[rb][nb][j] *= aj[j];
+          }
         }
       }
     }
-    stage(buf ^ 1, kt + 1);
+    stage(buf ^ 1, kt + KS);
     fetch(bt_far);
-    // O += P . V over the tile's two 32-token chunks, each V operand serving both row blocks;
-    // the sums against a column of ones. Chunk outermost: consecutive products of one
-    // accumulator are 8 RB + RB MFMAs apart. The V operands (i = 8 c + nb) are read
-    // PF_V_AHEAD products ahead of their use, so the LDS latency hides behind the MFMAs.
-    uint4 vq[PF_V_AHEAD];
+    if (real) {
+      // O += P . V over the tile's two 32-token chunks, each V operand serving both row blocks;
+      // the sums against a column of ones. Chunk outermost: consecutive products of one
+      // accumulator are 8 RB + RB MFMAs apart. The V operands (i = 8 c + nb) are read
+      // PF_V_AHEAD products ahead of their use, so the LDS latency hides behind the MFMAs.
+      uint4 vq[PF_V_AHEAD];
 #pragma unroll
-    for (int i = 0; i < PF_V_AHEAD; ++i) vq[i] = vread(buf, i);
+      for (int i = 0; i < PF_V_AHEAD; ++i) vq[i] = vread(buf, i);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int c = i >> 3, nb = i & 7;
-      const uint4 vop = vq[i % PF_V_AHEAD];
-      if (i + PF_V_AHEAD < 16) vq[i % PF_V_AHEAD] = vread(buf, i + PF_V_AHEAD);
+      for (int i = 0; i < 16; ++i) {
+        const int c = i >> 3, nb = i & 7;
+        const uint4 vop = vq[i % PF_V_AHEAD];
+        if (i + PF_V_AHEAD < 16) vq[i % PF_V_AHEAD] = vread(buf, i + PF_V_AHEAD);
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) acc[rb][nb] = tile::mfma16<DT>(pk[rb][c], vop, acc[rb][nb]);
-      if (nb == 7) {
+        for (int rb = 0; rb < RB; ++rb) acc[rb][nb] = tile::mfma16<DT>(pk[rb][c], vop, acc[rb][nb]);
+        if (nb == 7) {
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) lsum[rb] = tile::mfma16<DT>(pk[rb][c], ones, lsum[rb]);
+          for (int rb = 0; rb < RB; ++rb) lsum[rb] = tile::mfma16<DT>(pk[rb][c], ones, lsum[rb]);
+        }
       }
-    }
-    // keep that order through the machine scheduler (it would sink the reads to their uses):
-    // PF_V_AHEAD reads, then one read per RB products, then the rest of the products
-    __builtin_amdgcn_sched_group_barrier(0x100, PF_V_AHEAD, 0);
+      // keep that order through the machine scheduler (it would sink the reads to their uses):
+      // PF_V_AHEAD reads, then one read per RB products, then the rest of the products
+      __builtin_amdgcn_sched_group_barrier(0x100, PF_V_AHEAD, 0);
 #pragma unroll
-    for (int i = 0; i < 16 - PF_V_AHEAD; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, RB, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      for (int i = 0; i < 16 - PF_V_AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, RB, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, RB * (PF_V_AHEAD + 2), 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, RB * (PF_V_AHEAD + 2), 0);
     __syncthreads();
     bt_cur = bt_nxt;
     bt_nxt = bt_far;
     bt_far = bt_next_far;
+  }
+
+  if constexpr (KS == 2) {
+    // group 1's sums join group 0's: [value][thread] over the tile buffers, all read by now
+    static_assert(NW == 4, "64 + 10 floats per thread of a group in the K and V buffers");
+    float* xs = reinterpret_cast<float*>(&ks_all[0][0][0]);
+    float* ys = reinterpret_cast<float*>(&vs_all[0][0][0]);
+    constexpr int GT = 64 * NW;
+    __syncthreads();
+    if (kgrp == 1) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int nb = 0; nb < 8; ++nb) xs[((rb * 8 + nb) * 4 + j) * GT + tid] = acc[rb][nb][j];
+          ys[(rb * 4 + j) * GT + tid] = lsum[rb][j];
+        }
+        ys[(4 * RB + rb) * GT + tid] = m[rb];
+      }
+    }
+    __syncthreads();
+    if (kgrp == 1) return;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const float m1 = ys[(4 * RB + rb) * GT + tid];
+      const float mm = __builtin_elementwise_maximum(m[rb], m1);
+      const float f0 = m[rb] == mm ? 1.f : __builtin_amdgcn_exp2f((m[rb] - mm) * scale_log2);
+      const float f1 = m1 == mm ? 1.f : __builtin_amdgcn_exp2f((m1 - mm) * scale_log2);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float a = __shfl(f0, 4 * g4 + j, 64), c = __shfl(f1, 4 * g4 + j, 64);
+        lsum[rb][j] = lsum[rb][j] * a + ys[(rb * 4 + j) * GT + tid] * c;
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb)
+          acc[rb][nb][j] = acc[rb][nb][j] * a + xs[((rb * 8 + nb) * 4 + j) * GT + tid] * c;
+      }
+    }
   }
 
   // out = O / sum for rows 4 g4 + j of each block
@@ -456,37 +508,46 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
   const bool wide = 2 * total_q_rows >= int64_t(wide_ppt) * num_seqs &&
                     (ceil_div(total_q_rows, wide_ppt) + num_seqs) * Hkv >= 2 * int64_t(device_cus());
   const int ppt = (wide ? 8 : 4) * PF_WROWS / G;
+  // With no more items of four waves than compute units and tables of 768 keys or more, two groups
+  // of waves share an item's keys: its chain of tiles, which is the call's time then, is half as
+  // long, for a longer start and a merge. One sequence, 32/8 heads: 300 rows behind 1500 tokens
+  // 54.2 -> 45.0 us, 40 behind 1000 35.8 -> 31.7; 300 rows on their own 17.4 against 19.3.
+  const bool split =
+      !wide && bt_stride * PF_P >= 768 &&
+      (ceil_div(total_q_rows, 4 * PF_WROWS / G) + num_seqs) * Hkv <= device_cus();
   // work items: at most ceil(total rows / ppt) + one partial item per sequence
   const int64_t items = (ceil_div(total_q_rows, ppt) + num_seqs) * Hkv;
   const int64_t blocks = ceil_div(items, 8) * 8;
   if (blocks > 0x7fffffff)
     return fail(PIA_EINVAL, "paged_attention: too many query rows for the prefill kernel");
   const dim3 grid{unsigned(blocks), 1u, 1u};
-#define PIA_PF(GG, NW)                                                                         \
-  hipLaunchKernelGGL((paged_prefill_mfma<GG, NW, DT>), grid, dim3(64 * NW), 0, s,              \
+#define PIA_PF(GG, NW, KS)                                                                     \
+  hipLaunchKernelGGL((paged_prefill_mfma<GG, NW, KS, DT>), grid, dim3(64 * NW * KS), 0, s,     \
                      reinterpret_cast<uint16_t*>(out), reinterpret_cast<const uint16_t*>(q),   \
                      reinterpret_cast<const uint16_t*>(k_pages),                               \
                      reinterpret_cast<const uint16_t*>(v_pages), bt, bt_stride, kv_lens, cu_q, \
                      offsets, num_seqs, Hkv, num_pages, scale_log2)
-#define PIA_PF_G(NW)                  \
-  switch (G) {                        \
-    case 1: PIA_PF(1, NW); break;     \
-    case 2: PIA_PF(2, NW); break;     \
-    case 4: PIA_PF(4, NW); break;     \
-    default: PIA_PF(8, NW); break;    \
+#define PIA_PF_G(NW, KS)                  \
+  switch (G) {                            \
+    case 1: PIA_PF(1, NW, KS); break;     \
+    case 2: PIA_PF(2, NW, KS); break;     \
+    case 4: PIA_PF(4, NW, KS); break;     \
+    default: PIA_PF(8, NW, KS); break;    \
   }
-#define PIA_PF_D(NW)                           \
+#define PIA_PF_D(NW, KS)                       \
   if (dtype == PIA_DTYPE_F16) {                \
     constexpr int DT = PIA_DTYPE_F16;          \
-    PIA_PF_G(NW)                               \
+    PIA_PF_G(NW, KS)                           \
   } else {                                     \
     constexpr int DT = PIA_DTYPE_BF16;         \
-    PIA_PF_G(NW)                               \
+    PIA_PF_G(NW, KS)                           \
   }
   if (wide) {
-    PIA_PF_D(8);
+    PIA_PF_D(8, 1);
+  } else if (split) {
+    PIA_PF_D(4, 2);
   } else {
-    PIA_PF_D(4);
+    PIA_PF_D(4, 1);
   }
 #undef PIA_PF_D
 #undef PIA_PF_G
