@@ -7,7 +7,12 @@
 //   K: lane l loads vector 4 (n16 % 4) + n16 / 4 of rows d = 4 i + kd.
 //   V: lane l loads vectors 4 u + kd of rows d = 16 nb + n16.
 // Either load covers whole 128-byte lines: 4 consecutive K rows of each page (16-token pages:
-// 256 bytes per page in fp32, 128 in 16 bits), or 16 V rows of one page (two in 16 bits).
+// 256 bytes per page in fp32, 128 in 16 bits), or 16 V rows of one page (two in 16 bits). That is
+// the decode kernel's order, whose tiles come from HBM, once. The multi-row kernel, whose tiles
+// come from L2, takes K vector n16 and V vectors 4 kd + u instead (4 v + kd and 4 u + kd below
+// become 4 kd + v and 4 kd + u): its K loads then cost 0.8 times as much, neighbouring lanes
+// reading neighbouring vectors, while its V loads are spread over four pages each, which costs
+// nothing there. In the decode kernel that order measured 60.8 -> 106.7 us (32 sequences, fp32).
 //
 // fp32 storage, v_mfma_f32_16x16x4_f32 (A: lane l holds A[n16][kd]; B: B[kd][n16]; C: lane l
 // holds C[4 kd + v][n16]):

@@ -22,7 +22,10 @@
 //
 // Measured against paged_attention_tiled, which ran a workgroup per row: 2 sequences of 300..600
 // rows behind 0..512 tokens, 16/8 heads of 128, fp32:
-// 743 -> 116 us, and 98 us with the heads dealt to the XCDs.
+// 743 -> 116 us, 98 us with the heads dealt to the XCDs, 93 us with the K loads' lanes in the order
+// of their vectors (8 sequences of 1024 rows behind 3072, 28/4 heads, bf16: 1964 -> 1504 us). Two
+// 16-row blocks per wave, which halve the tile reads: 88 and 1535 us, and 28.6 against 23.0 us for
+// 2 short ones at head_dim 64; not kept.
 #include <algorithm>
 
 #include "attn_tiles.h"
@@ -150,7 +153,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
   const int64_t P4 = 4 * int64_t(P), P16 = 16 * int64_t(P);
   auto load_k = [&](uint4 (&kr)[16], int64_t o, int i0) {
     const int l = lane_now(), kd = l >> 4, n16 = l & 15;
-    const T* p = kpool + shfl64(o, 4 * (n16 & 3) + (n16 >> 2)) + (4 * i0 + kd) * int64_t(P);
+    const T* p = kpool + shfl64(o, n16) + (4 * i0 + kd) * int64_t(P);
 #pragma unroll
     for (int i = 0; i < 16; ++i) kr[i] = tile32::load16<false>(p + i * P4);
   };
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
     const int l = lane_now(), kd = l >> 4, n16 = l & 15;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-      const T* p = vpool + shfl64(o, 4 * (u0 + u) + kd) + n16 * int64_t(P);
+      const T* p = vpool + shfl64(o, 4 * kd + u0 + u) + n16 * int64_t(P);
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) vr[nb * NU + u] = tile32::load16<false>(p + nb * P16);
     }
@@ -202,7 +205,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
       }
       __builtin_amdgcn_sched_barrier(0);
 
-      // softmax of row n16: token TV (4 v + kd) + c of the tile is s[c][v]
+      // softmax of row n16: token TV (4 kd + v) + c of the tile is s[c][v]
       if constexpr (DT != PIA_DTYPE_F32) {
 #pragma unroll
         for (int c = 0; c < TV; ++c) s[c] *= scale_log2;
@@ -211,7 +214,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
         const int kd = lane_now() >> 4;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int n = min(__shfl(nv16, 4 * v + kd, 64), lim - (t * 16 + 4 * v + kd) * TV);
+          const int n = min(__shfl(nv16, 4 * kd + v, 64), lim - (t * 16 + 4 * kd + v) * TV);
 #pragma unroll
           for (int c = 0; c < TV; ++c) s[c][v] = c < n ? s[c][v] : -INFINITY;
         }
@@ -253,8 +256,8 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
           bool nf = false;
 #pragma unroll
           for (int u = 0; u < NU; ++u) {
-            const int n = __shfl(nv16, 4 * (u0 + u) + kd, 64);
-            const int own = kmin - (t * 16 + 4 * (u0 + u) + kd) * TV;  // tokens every row sees
+            const int n = __shfl(nv16, 4 * kd + u0 + u, 64);
+            const int own = kmin - (t * 16 + 4 * kd + u0 + u) * TV;  // tokens every row sees
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
               uint4& x = vr[nb * NU + u];
@@ -281,7 +284,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
         for (int u = 0; u < NU; ++u)
 #pragma unroll
           for (int c = 0; c < TV; ++c)
-            part[wave][n16 * TS + (4 * u + kd) * TV + c] = s[c][u0 + u];
+            part[wave][n16 * TS + (NU * kd + u) * TV + c] = s[c][u0 + u];
         int lim_j[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) lim_j[j] = __shfl(lim, 4 * kd + j, 64);
@@ -289,7 +292,7 @@ __global__ __launch_bounds__(64 * PR_WAVES, 2) void paged_attention_rows(
         __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
         for (int i = 0; i < 4 * NU * TV; ++i) {
-          const int x = 4 * u0 + i / TV, c = i % TV, tok = (t * 16 + x) * TV + c;
+          const int x = 4 * (i / TV / NU) + u0 + i / TV % NU, c = i % TV, tok = (t * 16 + x) * TV + c;
           if (c >= __builtin_amdgcn_readlane(nv16, x)) continue;
           const T* p = vpool + shfl64(off_cur, x) + c + n16 * int64_t(P);
 #pragma unroll
