@@ -347,6 +347,23 @@ int pia_moe_unpermute(void* out, const void* y, int64_t y_rows, const int32_t* r
 int pia_moe_sum_reduce(void* out, const void* in, int64_t num_tokens, int topk, int hidden_dim,
                        int dtype, void* stream);
 
+/* The routed gated-MLP FFN (reference: fused_experts_decode_impl,
+ * src/plastic_infer/moe/fused.py:276-359) as one call: pia_moe_align_block_size (blocks of 16),
+ * pia_moe_expert_gemm over w1 [E, 2 inter, hidden] with the activation, then over w2
+ * [E, hidden, inter], and pia_moe_sum_reduce into out [T, hidden]. x is [T, hidden] with row stride
+ * ldx. route_out [T, topk, hidden]: the routes' rows before the sum (rows of ids outside [0, E)
+ * are left as they are); NULL: kept in the workspace. out may be NULL when route_out is given (no
+ * sum), and may be x. act [T * topk, inter] with row stride ld_act, or NULL: kept in the workspace.
+ * workspace: 256-byte aligned, of pia_moe_ffn_workspace_bytes (own_act / own_route: whether act /
+ * route_out are NULL). */
+int64_t pia_moe_ffn_workspace_bytes(int64_t num_tokens, int topk, int num_experts, int hidden,
+                                    int inter, int dtype, int own_act, int own_route);
+int pia_moe_ffn(void* out, void* route_out, const void* x, int64_t ldx, const void* w1,
+                const void* w2, const float* topk_weights, const int32_t* topk_ids,
+                int64_t num_tokens, int topk, int num_experts, int hidden, int inter,
+                int activation, int weight_on_input, int dtype, void* act, int64_t ld_act,
+                void* workspace, int64_t workspace_bytes, void* stream);
+
 /* out = s / sqrt(mean(s^2) + eps) * weight over rows of n elements, s = x, or x + residual rounded
  * to the dtype and written to sum (a buffer of its own) when residual is given. The
  * reference's rms_norm (src/plastic_infer/exec/attention.py:77-79) with fp32 arithmetic and one

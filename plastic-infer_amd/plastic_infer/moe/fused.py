@@ -8,8 +8,8 @@
   FusedMoe                   :362-390 router + experts behind BaseMoeBackend
 All run as HIP kernels. The permute plan orders routes inside an expert by ascending flattened
 route index (deterministic; the reference's atomic-based order is not). Both FFN entry points
-share one plan-driven path: moe_align_block_size, the first expert GEMM with the activation
-fused into its epilogue, the second expert GEMM with the routing weight, moe_sum_reduce; the
+share one plan-driven native call (pia_moe_ffn): the plan of moe_align_block_size, the first expert
+GEMM with the activation fused into its epilogue, the second with the routing weight, the sum; the
 rounding points are the reference's (first GEMM output, activation output, second GEMM output
 and the sum are each rounded to the storage dtype; with fp32 storage there is no rounding).
 """
@@ -20,11 +20,11 @@ import torch
 
 from .. import _native as N
 from ..kernel.moe_ops import moe_align_block_size as _align
-from ..kernel.moe_ops import moe_expert_gemm, moe_sum_reduce, moe_topk
+from ..kernel.moe_ops import ACTIVATION_CODES, moe_topk
 from .base import BaseMoeBackend
 
-# Plan block of the expert GEMMs: the kernel takes 16 planned routes per work item, so the
-# finest block wastes the fewest padded rows when an expert serves only a few routes.
+# Plan block of the expert GEMMs (the native call's own): the kernel takes 16 planned routes per work
+# item, so the finest block wastes the fewest padded rows when an expert serves only a few routes.
 EXPERT_BLOCK_M = 16
 
 
@@ -91,34 +91,55 @@ def routed_ffn_routes(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
             or route_out.dtype != hidden_states.dtype:
         raise ValueError(f"route_out must be a contiguous [{M}, {k}, {H}] tensor of the "
                          "hidden dtype")
-    ids = topk_ids if topk_ids.dtype == torch.int32 else topk_ids.to(torch.int32)
-    weights = topk_weights.to(torch.float32).contiguous()
-    sorted_ids, expert_ids, npp = _align(ids, EXPERT_BLOCK_M, E)
-    dev = hidden_states.device
-    ws = torch.empty(N.query("pia_moe_expert_gemm_workspace_bytes", sorted_ids.numel(),
-                             EXPERT_BLOCK_M), dtype=torch.uint8, device=dev)
-    if act_buffer is None:
-        act_buffer = torch.empty(numel, two_i // 2, dtype=hidden_states.dtype, device=dev)
-    moe_expert_gemm(hidden_states, w1, weights, sorted_ids, expert_ids, npp, EXPERT_BLOCK_M,
-                    numel, k, activation=activation,
-                    mul_routed_weight=apply_router_weight_on_input, out=act_buffer, workspace=ws)
-    moe_expert_gemm(act_buffer, w2, weights, sorted_ids, expert_ids, npp, EXPERT_BLOCK_M, numel,
-                    1, activation=None, mul_routed_weight=not apply_router_weight_on_input,
-                    out=route_out.view(numel, H), workspace=ws)
+    if act_buffer is not None and (
+            act_buffer.dim() != 2 or act_buffer.stride(1) != 1 or act_buffer.shape[1] != two_i // 2
+            or act_buffer.shape[0] < numel or act_buffer.dtype != hidden_states.dtype):
+        raise ValueError(f"act_buffer must be [>= {numel}, {two_i // 2}] of the hidden dtype with "
+                         "unit column stride")
+    if hidden_states.stride(1) != 1 or hidden_states.shape[1] != w1.shape[2]:
+        raise ValueError(f"hidden_states must be [T, {w1.shape[2]}] with contiguous rows")
+    if w2.shape[0] < E or w2.shape[1:] != (H, two_i // 2) or two_i % 2 \
+            or not (w1.is_contiguous() and w2.is_contiguous()):
+        raise ValueError("w1 must be contiguous [E, 2 I, H] and w2 contiguous [E, H, I]")
+    if w1.dtype != hidden_states.dtype or w2.dtype != hidden_states.dtype:
+        raise ValueError("hidden_states, w1 and w2 must share a dtype")
+    if topk_weights.numel() != numel:
+        raise ValueError("topk_weights must hold one weight per route")
+    N.require_device(hidden_states, w1, w2, topk_weights, topk_ids, route_out,
+                     *(() if act_buffer is None else (act_buffer,)))
+    _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, apply_router_weight_on_input,
+         None, route_out, act_buffer)
     return route_out
+
+
+def _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, on_input, out, route_out=None,
+         act_buffer=None) -> None:
+    """The FFN of arguments already checked (pia_moe_ffn), every buffer not given in one
+    workspace."""
+    act = ACTIVATION_CODES.get(activation)
+    if act is None:
+        raise ValueError(f"Unsupported activation: {activation}")
+    M, H = hidden_states.shape
+    E, inter, k = w1.shape[0], w2.shape[2], topk_ids.shape[1]
+    ids = topk_ids.to(torch.int32).contiguous()
+    weights = topk_weights.to(torch.float32).contiguous()
+    dt, dev = N.dtype_code(hidden_states.dtype), hidden_states.device
+    ws_bytes = N.query("pia_moe_ffn_workspace_bytes", M, k, E, H, inter, dt,
+                       1 if act_buffer is None else 0, 1 if route_out is None else 0)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    N.call("pia_moe_ffn", N.ptr(out), N.ptr(route_out), hidden_states.data_ptr(),
+           hidden_states.stride(0), w1.data_ptr(), w2.data_ptr(), weights.data_ptr(),
+           ids.data_ptr(), M, k, E, H, inter, act, 1 if on_input else 0, dt, N.ptr(act_buffer),
+           0 if act_buffer is None else act_buffer.stride(0), ws.data_ptr(), ws_bytes,
+           N.stream_of(dev))
 
 
 def _routed_ffn(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
                 topk_weights: torch.Tensor, topk_ids: torch.Tensor, activation: str,
                 apply_router_weight_on_input: bool, out: torch.Tensor) -> torch.Tensor:
-    M, H = hidden_states.shape
-    k = topk_ids.shape[1]
-    if M * k == 0:
-        return out
-    route_out = torch.empty(M, k, H, dtype=hidden_states.dtype, device=hidden_states.device)
-    routed_ffn_routes(hidden_states, w1, w2, topk_weights, topk_ids, route_out, activation,
-                      apply_router_weight_on_input)
-    moe_sum_reduce(route_out, out)
+    if topk_ids.numel():
+        _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation,
+             apply_router_weight_on_input, out)
     return out
 
 

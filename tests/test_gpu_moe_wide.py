@@ -11,6 +11,8 @@ import torch
 import oracle.fused_experts as OF
 import oracle.moe_route as OM
 from plastic_infer.kernel import moe_align_block_size, moe_expert_gemm
+from plastic_infer.moe.fused import (
+    fused_experts_decode_impl, fused_experts_impl, routed_ffn_routes)
 
 pytestmark = pytest.mark.gpu
 
@@ -101,3 +103,36 @@ def test_one_launch_plan(dev, T, k, E, skew):
     assert np.array_equal(s.cpu().numpy(), rs)
     assert np.array_equal(e.cpu().numpy()[:rnpp // 16], re[:rnpp // 16])
     assert np.array_equal(pos.cpu().numpy(), rpos)
+
+
+@pytest.mark.parametrize("T,dtype,on_input", [(1, torch.float16, False), (37, torch.bfloat16, True),
+                                              (700, torch.bfloat16, False), (9, torch.float32, True)])
+def test_ffn_call(dev, T, dtype, on_input):
+    """The whole FFN call: strided hidden rows, a caller's activation buffer and route rows, routes
+    of no expert left alone, and the result over its own input; all the same bits."""
+    H, I, E, k = 264, 72, 9, 3
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H + 8, generator=g).to(dtype).to(dev)[:, :H]
+    w1 = (torch.randn(E, 2 * I, H, generator=g) * 0.05).to(dtype).to(dev)
+    w2 = (torch.randn(E, H, I, generator=g) * 0.05).to(dtype).to(dev)
+    tw, ids = torch.rand(T, k, generator=g).to(dev), torch.randint(-1, E, (T, k), generator=g)
+    ids = ids.to(torch.int32).to(dev)
+    routes = [torch.full((T, k, H), 7.0, dtype=dtype, device=dev) for _ in range(2)]
+    act = torch.empty(T * k, I + 8, dtype=dtype, device=dev)[:, :I]
+    routed_ffn_routes(x, w1, w2, tw, ids, routes[0], "gelu", on_input)
+    routed_ffn_routes(x, w1, w2, tw, ids, routes[1], "gelu", on_input, act_buffer=act)
+    assert torch.equal(routes[0], routes[1])
+    assert bool((routes[0][ids < 0] == 7.0).all())
+    ref, _, _ = OF.fused_experts(x.cpu(), w1.cpu(), w2.cpu(), tw.cpu(), ids.cpu().clamp_min(0),
+                                 "gelu", on_input, return_intermediate=True)
+    full = ids.clamp_min(0)
+    out = fused_experts_decode_impl(x.contiguous(), w1, w2, tw, full, "gelu", on_input)
+    err = (out.cpu().float() - ref.float()).abs().max() / ref.float().abs().max()
+    assert err < (2e-5 if dtype == torch.float32 else 1e-2)
+    xc = x.contiguous()
+    assert fused_experts_impl(xc, w1, w2, tw, full, "gelu", on_input) is xc
+    assert torch.equal(xc, out)
+    with pytest.raises(ValueError):
+        routed_ffn_routes(x, w1, w2[:, :, :64].contiguous(), tw, ids, routes[0], "gelu", on_input)
+    with pytest.raises(ValueError):
+        routed_ffn_routes(x, w1, w2, tw, ids, routes[0], "gelu", on_input, act_buffer=act[:, :64])
