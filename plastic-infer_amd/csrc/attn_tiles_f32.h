@@ -97,7 +97,8 @@ __device__ __forceinline__ uint32_t word(const uint4& x, int w) {
   return w == 0 ? x.x : w == 1 ? x.y : w == 2 ? x.z : x.w;
 }
 
-// s += K . Q^T over the 16 K rows of kr; q: the lane's q elements of those rows in LDS (fp32: 16
+// s += K . Q^T over the 16 K rows of kr (fp32: summed in fours of them, so that a score is not one
+// chain of D additions); q: the lane's q elements of those rows in LDS (fp32: 16
 // floats; 16-bit: 16 raw elements), 16-byte aligned
 template <int DT>
 __device__ __forceinline__ void qk(const uint4 (&kr)[16], const void* q,
@@ -108,10 +109,17 @@ __device__ __forceinline__ void qk(const uint4 (&kr)[16], const void* q,
     for (int i4 = 0; i4 < 4; ++i4) {
       const uint4 x = qv[i4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int c0 = 0; c0 < 4; c0 += 2) {
+        __builtin_amdgcn_sched_barrier(0);  // one pair of sums at a time (registers)
+        f32x4_t t[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          s[c] = mfma_f32(comp(kr[4 * i4 + j], c), comp(x, j), s[c]);
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            t[c] = mfma_f32(comp(kr[4 * i4 + j], c0 + c), comp(x, j), t[c]);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) s[c0 + c] += t[c];
+      }
     }
   } else {
 #pragma unroll
@@ -173,19 +181,33 @@ __device__ __forceinline__ void split3(const f32x4_t (&s)[8], int u, uint4 (&t)[
   for (int k = 0; k < 3; ++k) t[k] = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
 }
 
-// O += P . V over the V vectors u0 .. u0 + NU - 1 (vr[nb * NU + u - u0]), NB blocks of 16 d
+// O += P . V over the V vectors u0 .. u0 + NU - 1 (vr[nb * NU + u - u0]), NB blocks of 16 d. fp32:
+// the vectors' products are summed on their own first, two blocks at a time, so that a long
+// context is not one chain of additions.
 template <int DT, int NB, int NU>
 __device__ __forceinline__ void pv(const uint4 (&vr)[NB * NU], const f32x4_t (&p)[Vec<DT>::TV],
                                    int u0, f32x4_t (&acc)[NB]) {
+  if constexpr (DT == PIA_DTYPE_F32) {
 #pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    if constexpr (DT == PIA_DTYPE_F32) {
+    for (int n0 = 0; n0 < NB; n0 += 2) {
+      __builtin_amdgcn_sched_barrier(0);  // one pair at a time (registers)
+      f32x4_t t[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int u = 0; u < NU; ++u)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          acc[nb] = mfma_f32(p[c][u0 + u], comp(vr[nb * NU + u], c), acc[nb]);
-    } else {
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            t[j] = mfma_f32(p[c][u0 + u], comp(vr[(n0 + j) * NU + u], c), t[j]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        acc[n0 + j] += t[j];
+        asm volatile("" : "+v"(acc[n0 + j]));  // added now: delayed, the sums were spilled
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
       __builtin_amdgcn_sched_barrier(0);  // one set of terms at a time (registers)
       uint4 t[3];
       split3<DT>(p, u0 + u, t);
