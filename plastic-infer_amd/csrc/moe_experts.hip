@@ -905,13 +905,13 @@ __device__ __forceinline__ void direct_load(const __amdgpu_buffer_rsrc_t rsrc, u
   if constexpr (BYTES == 16) {
     if constexpr (NT)
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                   ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff) : "memory");
+                   ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff) : "memory", "m0");
     else
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                   ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff) : "memory");
+                   ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff) : "memory", "m0");
   } else {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                 ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff) : "memory");
+                 ::"s"(lds), "v"(off), "s"(rsrc), "s"(soff) : "memory", "m0");
   }
 }
 
