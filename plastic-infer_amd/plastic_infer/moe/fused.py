@@ -105,6 +105,8 @@ def routed_ffn_routes(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
         raise ValueError("hidden_states, w1 and w2 must share a dtype")
     if topk_weights.numel() != numel:
         raise ValueError("topk_weights must hold one weight per route")
+    if topk_ids.numel() < numel:
+        raise ValueError(f"topk_ids must hold the {numel} routes of hidden_states")
     N.require_device(hidden_states, w1, w2, topk_weights, topk_ids, route_out,
                      *(() if act_buffer is None else (act_buffer,)))
     _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, apply_router_weight_on_input,

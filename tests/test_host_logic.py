@@ -10,6 +10,7 @@ import random
 
 import numpy as np
 import pytest
+import torch
 
 import oracle.expert_copy as OC
 from plastic_infer.kv.chunk import (
@@ -18,6 +19,7 @@ from plastic_infer.kv.chunk import (
     longest_prefix_hits,
 )
 from plastic_infer.kv.paged import BlockTable, PageAllocator
+from plastic_infer.moe.fused import routed_ffn_routes
 from plastic_infer.store.resident import LruPool
 from plastic_infer.store.tiers import Tier
 
@@ -308,3 +310,13 @@ def test_staging_lru_follows_the_admission_rule(seed, n_slots, universe, calls):
         assert np.array_equal(victims, dst.astype(np.int64))
     lru.forget_range(0, n_slots)
     assert (lru.owner == -1).all() and not lru.slot_of
+
+
+def test_routed_ffn_refuses_fewer_ids_than_routes():
+    """The native call reads T * k ids, T from hidden_states: a shorter topk_ids is refused before
+    any pointer is passed on."""
+    T, k, E, H, I = 5, 2, 4, 16, 8
+    x, w1, w2 = torch.zeros(T, H), torch.zeros(E, 2 * I, H), torch.zeros(E, H, I)
+    tw, ids = torch.ones(T, k), torch.zeros(T - 1, k, dtype=torch.int32)
+    with pytest.raises(ValueError, match="topk_ids must hold the 10 routes"):
+        routed_ffn_routes(x, w1, w2, tw, ids, torch.zeros(T, k, H))
