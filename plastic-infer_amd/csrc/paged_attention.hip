@@ -449,7 +449,8 @@ __device__ __forceinline__ void sd_flush_appends(const int64_t (*rec)[2], int n_
 // first global step or -1, arr_ns its steps, arr_row = b * Hkv + h) are written; count them in
 // on their segments' counters and merge every segment whose last partial this is. Partial
 // layout per slot: G rows of [D unnormalised output, running max (log2 units), row sum]; a merge
-// takes GB of them at a time.
+// takes GB of them at a time. A row without keys (sum 0) is zeros; a NaN sum (a NaN or +inf score)
+// makes the row NaN, as in a segment that is not cut.
 template <int GB, int DT, int D = FD_D>
 __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
                                                     const int (&arr_ns)[2],
@@ -532,7 +533,7 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
 #pragma unroll
         for (int i = 0; i < ND; ++i)
           Elem<DT>::store(orow, int64_t(g0 + g) * D + 64 * i + lane,
-                          lt[g] > 0.f ? o[g][i] / lt[g] : 0.f);
+                          lt[g] == 0.f ? 0.f : o[g][i] / lt[g]);
       }
     }
   }
@@ -925,7 +926,7 @@ __global__ __launch_bounds__(64, 2) void paged_decode_stream(
 #pragma unroll
             for (int j = 0; j < 4; ++j)
               out[(row0 + g) * D + 32 * j + (lane >> 1)] =
-                  to16<DT>(lsum[g] > 0.f ? acc[j][g] / lsum[g] : 0.f);
+                  to16<DT>(lsum[g] == 0.f ? 0.f : acc[j][g] / lsum[g]);
         }
       } else {
         const int slot = seg_first < start ? 0 : 1;
@@ -1903,7 +1904,7 @@ __global__ __launch_bounds__(64) void paged_attention_generic(
 #pragma unroll
   for (int i = 0; i < DPL; ++i) {
     const int d = lane + 64 * i;
-    if (d < D) E::store(out, ooff + d, l > 0.f ? acc[i] / l : 0.f);
+    if (d < D) E::store(out, ooff + d, l == 0.f ? 0.f : acc[i] / l);
   }
 }
 

@@ -115,3 +115,29 @@ def test_decode_f32_infinite_values(dev, dtype):
     assert torch.equal(out[0].view(2, 4, 64), vp[0, :, :, 0].cpu().view(2, 1, 64).expand(-1, 4, -1))
     assert (out[1, :, 9] == float("inf")).all()
     assert out[1, :, torch.arange(64) != 9].isfinite().all()
+
+
+@pytest.mark.parametrize("dtype,D,P,G", [
+    (torch.float32, 128, 16, 2), (torch.bfloat16, 64, 16, 4), (torch.float16, 128, 32, 16),
+    (torch.bfloat16, 128, 16, 4), (torch.float16, 128, 16, 1), (torch.bfloat16, 128, 16, 8),
+    (torch.float32, 128, 16, 65)])
+def test_decode_nan_score_reaches_its_rows(dev, dtype, D, P, G):
+    """A NaN in an admissible key makes the rows of its kv head NaN, whether the sequence is cut over
+    waves (rows 0, 1: more steps than one wave's share) or not (row 2), and no other row."""
+    Hkv, lens, at = 2, [3000, 2900, 40, 700], [5, 2899, 3, None]
+    n_pages = [(n + P - 1) // P for n in lens]
+    bt = torch.zeros(len(lens), max(n_pages), dtype=torch.int32)
+    for b, n in enumerate(n_pages):
+        bt[b, :n] = torch.arange(n) + sum(n_pages[:b])
+    g = torch.Generator().manual_seed(G)
+    kp, vp = (torch.randn(sum(n_pages), Hkv, D, P, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(len(lens), Hkv * G, D, generator=g).to(dtype)
+    for b, t in enumerate(at):
+        if t is not None:
+            kp[bt[b, t // P], 0, 7, t % P] = float("nan")
+    out = paged_decode_attention(q.to(dev), kp.to(dev), vp.to(dev), bt.to(dev),
+                                 torch.tensor(lens, dtype=torch.int32, device=dev)).cpu()
+    out = out.view(len(lens), Hkv, G, D)
+    for b, t in enumerate(at):
+        assert out[b, 0].isnan().all() if t is not None else out[b, 0].isfinite().all(), b
+        assert out[b, 1].isfinite().all(), b
