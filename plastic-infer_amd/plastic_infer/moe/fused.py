@@ -98,7 +98,7 @@ def routed_ffn_routes(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
                          "unit column stride")
     if hidden_states.stride(1) != 1 or hidden_states.shape[1] != w1.shape[2]:
         raise ValueError(f"hidden_states must be [T, {w1.shape[2]}] with contiguous rows")
-    if w2.shape[0] < E or w2.shape[1:] != (H, two_i // 2) or two_i % 2 \
+    if w2.shape[1:] != (H, two_i // 2) or two_i % 2 \
             or not (w1.is_contiguous() and w2.is_contiguous()):
         raise ValueError("w1 must be contiguous [E, 2 I, H] and w2 contiguous [E, H, I]")
     if w1.dtype != hidden_states.dtype or w2.dtype != hidden_states.dtype:
@@ -109,6 +109,11 @@ def routed_ffn_routes(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
         raise ValueError(f"topk_ids must hold the {numel} routes of hidden_states")
     N.require_device(hidden_states, w1, w2, topk_weights, topk_ids, route_out,
                      *(() if act_buffer is None else (act_buffer,)))
+    E2 = w2.shape[0]
+    if E2 < E:   # an expert without a second matrix gives zero rows, as any id of no weights does
+        ids = topk_ids.reshape(-1)[:numel].view(M, k, 1)
+        route_out.masked_fill_((ids >= E2) & (ids <= E), 0)
+        w1 = w1[:E2]
     _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, apply_router_weight_on_input,
          None, route_out, act_buffer)
     return route_out

@@ -136,3 +136,24 @@ def test_ffn_call(dev, T, dtype, on_input):
         routed_ffn_routes(x, w1, w2[:, :, :64].contiguous(), tw, ids, routes[0], "gelu", on_input)
     with pytest.raises(ValueError):
         routed_ffn_routes(x, w1, w2, tw, ids, routes[0], "gelu", on_input, act_buffer=act[:, :64])
+
+
+@pytest.mark.parametrize("T", [3, 400])
+def test_ffn_fewer_second_matrices(dev, T):
+    """w2 with fewer experts than w1: the experts it lacks (and the id one past w1's) give zero rows,
+    the others the rows of a call with all of w2, routes of no expert stay as they are."""
+    H, I, E, E2, k = 128, 64, 6, 4, 2
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    w1 = (torch.randn(E, 2 * I, H, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    w2 = (torch.randn(E, H, I, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    tw = torch.rand(T, k, generator=g).to(dev)
+    ids = torch.randint(-1, E + 1, (T, k), generator=g).to(torch.int32).to(dev)
+    full, part = (torch.full((T, k, H), 7.0, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    routed_ffn_routes(x, w1, w2, tw, ids, full)
+    routed_ffn_routes(x, w1, w2[:E2].contiguous(), tw, ids, part)
+    assert bool((part[ids < 0] == 7.0).all())
+    assert not bool(part[ids >= E2].any())
+    held = (ids >= 0) & (ids < E2)
+    err = (part[held].float() - full[held].float()).abs().max()
+    assert err <= 2.0 ** -7 * full[held].float().abs().max()   # one rounding step: other sum order
