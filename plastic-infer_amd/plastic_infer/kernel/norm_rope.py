@@ -2,12 +2,14 @@
 
 The formulas of exec.attention's rms_norm and RoPE helpers (reference:
 src/plastic_infer/exec/attention.py:53-95) with fp32 arithmetic and one rounding of the result.
-Tensors the kernels do not take (dtypes that differ, non-contiguous rows) go through those helpers.
+Tensors the kernels do not take (dtypes that differ, non-contiguous rows, values that autograd
+follows: the kernels record nothing for it) go through those helpers.
 """
 
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _native as N
 
@@ -15,7 +17,11 @@ EPS = 1e-5   # of the reference's rms_norm
 
 
 def _fits(*tensors: torch.Tensor) -> bool:
-    """Contiguous device tensors of one dtype that the kernels are built for."""
+    """Contiguous device tensors of one dtype that the kernels are built for, with no derivative
+    to be taken of them in either mode (inside a dual level any of them may carry a tangent)."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors) \
+            or getattr(forward_ad, "_current_level", -1) >= 0:
+        return False
     dt = tensors[0].dtype
     return dt in (torch.bfloat16, torch.float16, torch.float32) and all(
         t.dtype == dt and t.is_contiguous() and t.device == tensors[0].device for t in tensors) \
