@@ -110,26 +110,34 @@ def kv_gather(k_pages: torch.Tensor, v_pages: torch.Tensor, block_tables: torch.
 
 def decode_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
                            page_size: int, max_pages_per_seq: int) -> int:
-    """Scratch bytes paged_decode_attention needs for these shapes (0 if none)."""
+    """Bytes of the workspace that the decode calls take from their caller for these shapes; 0: they
+    take none (and leave one that is passed alone). Calls that share a workspace must be ordered on
+    one stream: a launch keeps its partials and arrival counters in it."""
     return N.query("pia_paged_decode_workspace_bytes", num_seqs, num_heads, num_kv_heads,
                    head_dim, page_size, max_pages_per_seq)
 
 
 def _decode_scratch(q: torch.Tensor, Hkv: int, P: int, max_pages: int,
                     workspace: torch.Tensor | None) -> tuple[torch.Tensor | None, int]:
-    """(workspace, its bytes) of a decode call: the caller's where it is large enough for the
-    call's kernel, else one allocated for the call; (None, 0) where no kernel takes one."""
+    """(scratch, its bytes) of a decode call: where decode_workspace_bytes is not 0, the caller's
+    workspace if it is large enough. The other shapes of the fp32-precision kernel take scratch of
+    their own for each call and leave a workspace alone: their callers, told that they need none, may
+    share one between streams or hold it anywhere. Without memory for it they run the kernel that
+    takes none."""
     B, Hq, D = q.shape
     need = decode_workspace_bytes(B, Hq, Hkv, D, P, max_pages)
-    if not need:
-        need = N.query("pia_paged_decode_split_scratch_bytes", Hq, Hkv, D, P,
-                       N.dtype_code(q.dtype))
+    if need:
+        have = 0 if workspace is None else workspace.numel() * workspace.element_size()
+        if have < need:
+            return torch.empty(need, dtype=torch.uint8, device=q.device), need
+        return workspace, have
+    need = N.query("pia_paged_decode_split_scratch_bytes", Hq, Hkv, D, P, N.dtype_code(q.dtype))
     if not need:
         return None, 0
-    have = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    if have < need:
+    try:
         return torch.empty(need, dtype=torch.uint8, device=q.device), need
-    return workspace, have
+    except torch.OutOfMemoryError:
+        return None, 0
 
 
 def paged_decode_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
@@ -138,7 +146,9 @@ def paged_decode_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
                            workspace: torch.Tensor | None = None) -> torch.Tensor:
     """One decode query row per sequence. q: [B, Hq, D]; block_tables int32 [B, max_pages];
     context_lens int32 [B] (tokens including the newest). Returns [B, Hq, D] in q's dtype.
-    Head hq reads kv head hq // (Hq // Hkv); scale defaults to 1/sqrt(D)."""
+    Head hq reads kv head hq // (Hq // Hkv); scale defaults to 1/sqrt(D).
+    workspace: device memory of decode_workspace_bytes, kept between calls that are ordered on one
+    stream; allocated for the call where none (or too little) is given."""
     dev = N.require_device(q, k_pages, v_pages, block_tables, context_lens,
                            names=("q", "k_pages", "v_pages", "block_tables", "context_lens"))
     _check_pool(k_pages, v_pages)

@@ -16,6 +16,7 @@ import torch
 
 from plastic_infer import _native as N
 from plastic_infer.kernel import paged_decode_append_attention, paged_decode_attention
+from plastic_infer.kernel.paged_kv import decode_workspace_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -141,3 +142,43 @@ def test_decode_nan_score_reaches_its_rows(dev, dtype, D, P, G):
     for b, t in enumerate(at):
         assert out[b, 0].isnan().all() if t is not None else out[b, 0].isfinite().all(), b
         assert out[b, 1].isfinite().all(), b
+
+
+def _small_call(dev, dtype, D, P):
+    g = torch.Generator().manual_seed(D)
+    kp, vp = (torch.randn(30, 2, D, P, generator=g).to(dtype).to(dev) for _ in range(2))
+    q = torch.randn(2, 8, D, generator=g).to(dtype).to(dev)
+    bt = torch.arange(30, dtype=torch.int32, device=dev).view(2, 15)
+    return q, kp, vp, bt, torch.tensor([201, 37], dtype=torch.int32, device=dev)
+
+
+@pytest.mark.parametrize("dtype,D,P", [(torch.float32, 128, 32), (torch.bfloat16, 64, 16)])
+def test_decode_f32_leaves_the_callers_workspace(dev, dtype, D, P):
+    """decode_workspace_bytes is 0 for these shapes: a workspace passed all the same (one a program
+    shares between streams, say) is not written."""
+    args = _small_call(dev, dtype, D, P)
+    assert decode_workspace_bytes(2, 8, 2, D, P, 15) == 0
+    assert N.query("pia_paged_decode_split_scratch_bytes", 8, 2, D, P, N.dtype_code(dtype)) > 0
+    ws = torch.full((1 << 26,), 0xAB, dtype=torch.uint8, device=dev)
+    out = paged_decode_attention(*args, workspace=ws)
+    assert bool((ws == 0xAB).all())
+    assert torch.equal(out, paged_decode_attention(*args))
+
+
+@pytest.mark.parametrize("dtype,D,P", [(torch.float32, 128, 32), (torch.bfloat16, 64, 16)])
+def test_decode_f32_without_memory_for_scratch(dev, dtype, D, P, monkeypatch):
+    """A pool that leaves no memory for the scratch: the kernel that takes none runs."""
+    args = _small_call(dev, dtype, D, P)
+    want = paged_decode_attention(*args)
+    empty = torch.empty
+
+    def none_left(*a, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no memory left")
+        return empty(*a, **kw)
+
+    monkeypatch.setattr(torch, "empty", none_left)
+    got = paged_decode_attention(*args)
+    monkeypatch.undo()
+    diff = (got.double() - want.double()).abs()   # both within the bars above of the exact result
+    assert (diff <= 2.02 * ROUNDOFF[dtype] * want.double().abs() + 2 * 4e-6 * 4.0).all()
