@@ -30,6 +30,7 @@
 //    time (lane = key for QK, lane = head-dim element for PV).
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
 #include <mutex>
 #include <random>
 #include <type_traits>
@@ -289,14 +290,19 @@ using PoolIn = std::conditional_t<APPEND, const uint16_t*, const uint16_t* __res
 // from another XCD, and that read was measured 0.4 % faster than after ordinary stores.
 // Arrivals of the n waves that hold partials of a cut segment: the segment's counter holds
 // (token << 16 | count) where token identifies the launch (the upper 48 bits, from the host, a
-// fresh value per launch). Every wave of the segment first makes sure that the counter carries
-// the token (sd_install, at the start of its range, under its first loads: a count under
-// another token is stale, from an earlier launch or a workspace never used before), then counts
-// itself in with one atomic add after its range. The n-th arrival merges; it also leaves the
-// count at 0 under this token, so a replay of the same launch (a graph) starts from zero again.
-// Workspace contents collide with a token with probability 2^-48. (Counting in with a
-// compare-and-swap loop instead costs a round trip per lost race: one sequence of 3001 tokens,
-// 24 pieces per head that end together, took 24.4 us with the loop and 17.8 us with this.)
+// fresh value per launch); a count under another token is stale (an earlier launch, or a
+// workspace never used before). A wave counts itself in after its range: where it sees the token,
+// with one atomic add, which no other wave's can make it repeat; else by exchanging the stale value
+// for the token and its own count, and if another wave was first, with that add. The n-th arrival
+// merges; it also leaves the count at 0 under this token, so a replay of the same launch (a graph)
+// starts from zero again. Workspace contents collide with a token with probability 2^-48.
+// The waves of a launch with one step for each pair of them end together and have time before that:
+// there a segment of SD_INSTALL_PIECES or more gets its token at their start (sd_install), under
+// their loads, and only the add is left at the end. (Counting in with a compare-and-swap loop costs
+// a round trip per lost race; the token put in at the start of every range, whatever its length,
+// costs the others a second cursor search and an atomic ahead of their loads. One sequence of 3001
+// tokens, 24 pieces: loop 24.1 us, start 17.9, now 17.2; 16 sequences of 2000:
+// 34.0, 35.4, 33.0.)
 // Device-coherent partial stores and loads (sc1: through the XCD's L2 to memory).
 __device__ __forceinline__ void sd_store(float* p, float v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -305,7 +311,21 @@ __device__ __forceinline__ float sd_load(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ bool sd_arrive(uint64_t* ctr, uint64_t token, int n) {
+__device__ __forceinline__ bool sd_has_token(uint64_t v, uint64_t token) {
+  return (v >> 16) == (token >> 16);
+}
+
+// The launch's token onto a counter last seen holding `old`: only waves of this launch touch the
+// counter, so where the exchange fails another of them has put the token there (and perhaps
+// counted itself in).
+__device__ __forceinline__ bool sd_install(uint64_t* ctr, uint64_t old, uint64_t value) {
+  return __hip_atomic_compare_exchange_strong(ctr, &old, value, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Arrival on a counter last seen holding `seen`; true for the n-th of n >= 2.
+__device__ __forceinline__ bool sd_arrive(uint64_t* ctr, uint64_t seen, uint64_t token, int n) {
+  if (!sd_has_token(seen, token) && sd_install(ctr, seen, token | 1u)) return false;
   const uint64_t prev = __hip_atomic_fetch_add(ctr, uint64_t(1), __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
   if (int(prev & 0xffffu) + 1 < n) return false;
@@ -313,17 +333,15 @@ __device__ __forceinline__ bool sd_arrive(uint64_t* ctr, uint64_t token, int n) 
   return true;
 }
 
-// The launch's token onto a counter last seen holding `old`, before any arrival of this wave:
-// only waves of this launch touch the counter, so where the exchange fails another of them has
-// installed the token (and perhaps counted itself in).
-__device__ __forceinline__ void sd_install(uint64_t* ctr, uint64_t old, uint64_t token) {
-  if ((old >> 16) != (token >> 16))
-    __hip_atomic_compare_exchange_strong(ctr, &old, token, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-}
-
 __device__ __forceinline__ uint64_t* sd_counters(int32_t* ws_meta) {
   return reinterpret_cast<uint64_t*>((reinterpret_cast<uintptr_t>(ws_meta) + 7) & ~uintptr_t(7));
+}
+
+// Pieces of a segment (its steps, in a launch with one step per pair of waves) from which its
+// counter gets the token ahead of the waves' loads.
+constexpr int SD_INSTALL_PIECES = 8;
+__device__ __forceinline__ bool sd_installs_first(int Dp, int ns) {
+  return Dp == 1 && ns >= SD_INSTALL_PIECES;
 }
 
 // Step prefix of the batch, built by every wave in its own LDS copy: seq_q[b] = steps (of STEP
@@ -464,13 +482,21 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
   const int inc = Ce < Dp ? 1 : 2;  // odd waves hold no steps when pairs have one step
   __builtin_amdgcn_s_waitcnt(0);  // this wave's partial stores have completed before its count
   bool merge[2] = {false, false};
+  int c0[2] = {0, 0}, c1[2] = {0, 0};
+  uint64_t seen[2] = {token, token};
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     if (arr_first[k] < 0) continue;
-    const int c0 = stream_range_of(arr_first[k], Dp, Ce);
-    const int c1 = stream_range_of(arr_first[k] + arr_ns[k] - 1, Dp, Ce);
+    c0[k] = stream_range_of(arr_first[k], Dp, Ce);
+    c1[k] = stream_range_of(arr_first[k] + arr_ns[k] - 1, Dp, Ce);
+    if (lane == 0 && !sd_installs_first(Dp, arr_ns[k]))
+      seen[k] = __hip_atomic_load(ctr + c0[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (arr_first[k] < 0) continue;
     int last = 0;
-    if (lane == 0) last = sd_arrive(ctr + c0, token, (c1 - c0) / inc + 1) ? 1 : 0;
+    if (lane == 0) last = sd_arrive(ctr + c0[k], seen[k], token, (c1[k] - c0[k]) / inc + 1) ? 1 : 0;
     merge[k] = __builtin_amdgcn_readfirstlane(last) != 0;
   }
   if (!merge[0] && !merge[1]) return;
@@ -479,15 +505,13 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
     if (!merge[k]) continue;
     // one online pass over the pieces in wave order (slot 1 of the first wave, slot 0 of the
     // rest)
-    const int c0 = stream_range_of(arr_first[k], Dp, Ce);
-    const int c1 = stream_range_of(arr_first[k] + arr_ns[k] - 1, Dp, Ce);
     const int b = arr_row[k] / Hkv, h = arr_row[k] - b * Hkv;
     typename Elem<DT>::T* orow = out + (int64_t(b) * Hkv * G + int64_t(h) * G) * D;
     for (int g0 = 0; g0 < G; g0 += GB) {
       float M[GB], o[GB][ND], lt[GB];
 #pragma unroll
       for (int g = 0; g < GB; ++g) {
-        M[g] = -INFINITY;
+        M[g] = -FLT_MAX;
         lt[g] = 0.f;
 #pragma unroll
         for (int i = 0; i < ND; ++i) o[g][i] = 0.f;
@@ -495,13 +519,13 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
       // pieces eight (GB <= 4), four or two at a time: their loads in flight together, folded
       // in order
       constexpr int PB = GB <= 4 ? 8 : GB <= 8 ? 4 : 2;
-      for (int cb = c0; cb <= c1; cb += PB * inc) {
+      for (int cb = c0[k]; cb <= c1[k]; cb += PB * inc) {
         float mc[PB][GB], lc[PB][GB], a[PB][GB][ND];
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
           const int c = cb + u * inc;
-          if (c > c1) continue;
-          const float* pp = ws_part + ((int64_t(c) * 2 + (c == c0 ? 1 : 0)) * G + g0) * (D + 2);
+          if (c > c1[k]) continue;
+          const float* pp = ws_part + ((int64_t(c) * 2 + (c == c0[k] ? 1 : 0)) * G + g0) * (D + 2);
 #pragma unroll
           for (int g = 0; g < GB; ++g) {
             if (g0 + g >= G) continue;
@@ -513,13 +537,15 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
         }
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
-          if (cb + u * inc > c1) continue;
+          if (cb + u * inc > c1[k]) continue;
 #pragma unroll
           for (int g = 0; g < GB; ++g) {
             if (g0 + g >= G) continue;
-            const float mn = fmaxf(M[g], mc[u][g]);
-            const float fo = M[g] == mn ? 1.f : fast_exp2(M[g] - mn);
-            const float fc = mc[u][g] == mn ? 1.f : fast_exp2(mc[u][g] - mn);
+            // a piece without a key has max -inf: finite here, so that no (-inf) - (-inf) arises
+            // (as selects on equal maxima in this chain: 17.4 -> 18.3 us at 3001 tokens)
+            const float mp = fmaxf(mc[u][g], -FLT_MAX);
+            const float mn = fmaxf(M[g], mp);
+            const float fo = fast_exp2(M[g] - mn), fc = fast_exp2(mp - mn);
             lt[g] = lt[g] * fo + lc[u][g] * fc;
 #pragma unroll
             for (int i = 0; i < ND; ++i) o[g][i] = o[g][i] * fo + a[u][g][i] * fc;
@@ -539,28 +565,20 @@ __device__ __forceinline__ void sd_arrive_and_merge(const int (&arr_first)[2],
   }
 }
 
-// The counters of the (at most two) cut segments of a wave's range: read by begin() ahead of the
-// range's first loads, given the launch's token by finish() behind them.
-struct SegmentCounters {
-  uint64_t* ctr[2] = {nullptr, nullptr};
-  uint64_t old[2] = {0, 0};
+// The counter of the segment of a one-step range, where it gets its token at the start: read by
+// begin() ahead of the range's loads, given the token by finish() behind them.
+struct SegmentCounter {
+  uint64_t* ctr = nullptr;
+  uint64_t old = 0;
 
-  __device__ __forceinline__ void begin(const StreamPlan& plan, const StreamCursor& first, int start,
-                                        int end, int Dp, int Ce, int32_t* ws_meta, int lane) {
-    uint64_t* base = sd_counters(ws_meta);
-    if (first.ls > 0) ctr[0] = base + stream_range_of(start - first.ls, Dp, Ce);
-    const StreamCursor last = plan.seg_of(end - 1);
-    const int f = end - 1 - last.ls;  // first step of the range's last segment
-    if (f >= start && f + last.ns > end) ctr[1] = base + stream_range_of(f, Dp, Ce);
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      if (ctr[k] && lane == 0)
-        old[k] = __hip_atomic_load(ctr[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __device__ __forceinline__ void begin(const StreamCursor& cur, int start, int Dp, int Ce,
+                                        int32_t* ws_meta, int lane) {
+    if (!sd_installs_first(Dp, cur.ns) || lane != 0) return;
+    ctr = sd_counters(ws_meta) + stream_range_of(start - cur.ls, Dp, Ce);
+    old = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __device__ __forceinline__ void finish(uint64_t token, int lane) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-      if (ctr[k] && lane == 0) sd_install(ctr[k], old[k], token);
+  __device__ __forceinline__ void finish(uint64_t token) {
+    if (ctr && !sd_has_token(old, token)) sd_install(ctr, old, token);
   }
 };
 
@@ -663,14 +681,14 @@ __global__ __launch_bounds__(64, 2) void paged_decode_stream(
     QRows q0;
     load_q(cur, q0);
     bt_cur = load_bt(cur);
-    SegmentCounters counters;
-    counters.begin(plan, cur, start, end, Dp, Ce, ws_meta, lane);
+    SegmentCounter counter;
+    counter.begin(cur, start, Dp, Ce, ws_meta, lane);
     const uint16_t* kp = kbase + int64_t(cur.h) * TILE + page_ok(bt_cur) * page_stride;
 #pragma unroll
     for (int i = 0; i < 16; ++i) bufA[i] = load16_nt(kp + 64 * i);
 #pragma unroll
     for (int i = 0; i < 16; ++i) bufB[i] = load16_nt(kp + 64 * (16 + i));
-    counters.finish(token, lane);
+    counter.finish(token);
     stage_q(q0);
     __syncthreads();
   }
@@ -1219,12 +1237,12 @@ __global__ __launch_bounds__(64, 1) void paged_decode_mfma(
   int arr_first[2] = {-1, -1}, arr_ns[2] = {0, 0}, arr_row[2] = {0, 0};
   load_q(cur, qreg);
   int bt_cur = load_bt(cur);
-  SegmentCounters counters;
-  counters.begin(plan, cur, start, end, Dp, Ce, ws_meta, lane);
+  SegmentCounter counter;
+  counter.begin(cur, start, Dp, Ce, ws_meta, lane);
   uint4 bufA[16], bufB[16];
   load_k(bufA, cur.h, bt_cur, 0);
   load_k(bufB, cur.h, bt_cur, 1);
-  counters.finish(token, lane);
+  counter.finish(token);
 
   for (;;) {
     {  // issue priority from progress: quartile 0 of the range -> 3, quartile 3 -> 0
@@ -1573,13 +1591,13 @@ __global__ __launch_bounds__(64, 2) void paged_decode_f32(
   int bt_cur = load_bt(cur), bt_nxt = load_bt(nxt);
   int64_t off_cur;
   {
-    SegmentCounters counters;
-    counters.begin(plan, cur, start, end, Dp, Ce, ws_meta, lane);
+    SegmentCounter counter;
+    counter.begin(cur, start, Dp, Ce, ws_meta, lane);
     off_cur = vec_off(cur, bt_cur);
     load_k(bufA, off_cur, 0);
     if constexpr (D == 128) load_k(bufB, off_cur, 16);
     else load_v(bufB, off_cur, 0);
-    counters.finish(token, lane);
+    counter.finish(token);
     for (int i = lane; i < 64 * QS; i += 64) qs[i] = T(0);  // rows G..15 stay zero
     wave_sync();
     stage_q(cur);

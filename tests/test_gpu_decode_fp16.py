@@ -18,6 +18,7 @@ import torch
 
 import oracle.paged_kv as OP
 from plastic_infer.kernel import paged_decode_append_attention, paged_decode_attention
+from plastic_infer.kernel.paged_kv import decode_workspace_bytes
 from test_gpu_append_decode import _case, _check
 from test_gpu_attention import oracle_max_err_all_rows, qwen3_8b_b256_inputs
 
@@ -95,3 +96,34 @@ def test_fp16_append_qwen3_8b_b256_full_shape(dev):
     del kb, vb
     worst = oracle_max_err_all_rows(out.cpu(), q, kp, vp, bt, lens, n_pages, P)
     assert worst <= FP16_TOL, worst
+
+
+@pytest.mark.parametrize("lens", [
+    [130], [900], [1000], [3001],           # 2, 8, 8 and 24 pieces per head, each wave one step
+    [700, 5, 1100, 129, 0, 2000],           # fewer and more than eight pieces in one launch
+    [2000] * 24,                            # several steps a wave, both ends of its range cut
+])
+@pytest.mark.parametrize("dtype,G", [(torch.float16, 4), (torch.bfloat16, 8), (torch.float32, 2)])
+def test_arrivals_from_any_workspace(dev, dtype, G, lens):
+    """Cut segments are merged once whatever the counters hold: a workspace of any content, and the
+    same one after calls of other shapes. Every call gives the same bits; with the tolerance of the
+    files of the three kernels against the oracle."""
+    Hkv = 8
+    need = sum((n + 15) // 16 for n in lens) + 8
+    q, kp, vp, bt, lens_t, _, _ = _case(80 + G, lens, Hkv * G, Hkv, need, dtype=dtype)
+    args = [x.to(dev) for x in (q, kp, vp, bt, lens_t)]
+    size = decode_workspace_bytes(len(lens), Hkv * G, Hkv, 128, 16, bt.shape[1])
+    g = torch.Generator(device=dev).manual_seed(G)
+    outs = [paged_decode_attention(*args)]
+    for fill in (0, 0xFF, None):
+        ws = torch.randint(0, 256, (size,), generator=g, device=dev, dtype=torch.uint8) \
+            if fill is None else torch.full((size,), fill, dtype=torch.uint8, device=dev)
+        for _ in range(3):
+            outs.append(paged_decode_attention(*args, workspace=ws))
+            paged_decode_attention(args[0][:1], *args[1:3], args[3][:1], args[4][:1], workspace=ws)
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
+    live = lens_t > 0
+    ref = OP.decode_batch(q[live], kp, vp, bt[live].clamp(min=0), lens_t[live], 16)
+    tol = {torch.float16: FP16_TOL, torch.bfloat16: 2e-2, torch.float32: 1e-5}[dtype]
+    assert (outs[0].cpu()[live].float() - ref.float()).abs().max().item() <= tol
