@@ -16,6 +16,7 @@ KV pools are [num_pages, num_kv_heads, head_dim, page_size]; all tensors live on
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -117,25 +118,32 @@ def decode_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, hea
                    head_dim, page_size, max_pages_per_seq)
 
 
-def _decode_scratch(q: torch.Tensor, Hkv: int, P: int, max_pages: int,
+@functools.lru_cache(maxsize=256)
+def _scratch_needs(Hq: int, Hkv: int, D: int, P: int, dtype: int, device: int) -> tuple[int, int]:
+    """(decode_workspace_bytes of any batch, scratch of the fp32-precision kernel), once per shape:
+    the two library queries cost as much as a short call's launch (2.8 us)."""
+    return (decode_workspace_bytes(1, Hq, Hkv, D, P, 1),
+            N.query("pia_paged_decode_split_scratch_bytes", Hq, Hkv, D, P, dtype))
+
+
+def _decode_scratch(q: torch.Tensor, Hkv: int, P: int,
                     workspace: torch.Tensor | None) -> tuple[torch.Tensor | None, int]:
     """(scratch, its bytes) of a decode call: where decode_workspace_bytes is not 0, the caller's
     workspace if it is large enough. The other shapes of the fp32-precision kernel take scratch of
     their own for each call and leave a workspace alone: their callers, told that they need none, may
     share one between streams or hold it anywhere. Without memory for it they run the kernel that
     takes none."""
-    B, Hq, D = q.shape
-    need = decode_workspace_bytes(B, Hq, Hkv, D, P, max_pages)
+    need, own = _scratch_needs(q.shape[1], Hkv, q.shape[2], P, N.dtype_code(q.dtype),
+                               q.device.index)
     if need:
         have = 0 if workspace is None else workspace.numel() * workspace.element_size()
         if have < need:
             return torch.empty(need, dtype=torch.uint8, device=q.device), need
         return workspace, have
-    need = N.query("pia_paged_decode_split_scratch_bytes", Hq, Hkv, D, P, N.dtype_code(q.dtype))
-    if not need:
+    if not own:
         return None, 0
     try:
-        return torch.empty(need, dtype=torch.uint8, device=q.device), need
+        return torch.empty(own, dtype=torch.uint8, device=q.device), own
     except torch.OutOfMemoryError:
         return None, 0
 
@@ -172,7 +180,7 @@ def paged_decode_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
         raise ValueError("out must be a contiguous [B, Hq, D] tensor of q's dtype")
     if B == 0:
         return out
-    workspace, ws_bytes = _decode_scratch(q, Hkv, P, block_tables.shape[1], workspace)
+    workspace, ws_bytes = _decode_scratch(q, Hkv, P, workspace)
     scale = (1.0 / math.sqrt(D)) if scale is None else float(scale)
     N.call("pia_paged_decode_attention", out.data_ptr(), q.data_ptr(), q.stride(0),
            k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
@@ -221,7 +229,7 @@ def paged_decode_append_attention(q: torch.Tensor, k_pages: torch.Tensor, v_page
         raise ValueError("out must be a contiguous [B, Hq, D] tensor of q's dtype")
     if B == 0:
         return out
-    workspace, ws_bytes = _decode_scratch(q, Hkv, P, block_tables.shape[1], workspace)
+    workspace, ws_bytes = _decode_scratch(q, Hkv, P, workspace)
     scale = (1.0 / math.sqrt(D)) if scale is None else float(scale)
     N.call("pia_paged_decode_append_attention", out.data_ptr(), q.data_ptr(), q.stride(0),
            k_pages.data_ptr(), v_pages.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
