@@ -42,7 +42,8 @@
 // block-table id is outside the pool) score -inf; their V words are zeros from the loads.
 //
 // Few items with many keys: two groups of four waves take every other tile of an item's keys, each
-// with its own buffers, maxima and sums, and meet in LDS at the end (template parameter KS).
+// with its own buffers, maxima and sums, and meet in LDS at the end (template parameter KS). An
+// item of such a call with fewer than PF_SPLIT_TILES tiles is the first group's; the second ends.
 //
 // Work list: by kv head, sequence, position tile (the last tiles of a sequence, which see the most
 // keys when causal, first), with the heads dealt to the XCDs (xcd_item), so the ~64 workgroups
@@ -64,6 +65,8 @@ constexpr int PF_WROWS = 16 * PF_RB;  // (position, head) rows per wave
 constexpr int PF_KT = 64;             // keys per tile: four pages
 constexpr int PF_MAX_SEQS = 1024;     // sequences per launch (tile prefix in LDS)
 constexpr int PF_V_AHEAD = 4;         // V operand reads in flight ahead of the P . V products
+constexpr int PF_SPLIT_TILES = 6;     // tiles of an item from which two wave groups share its keys,
+constexpr int PF_SPLIT_TABLE = 512;   // in calls whose tables hold at least this many keys
 // word 3 of a raw (stride 0) buffer descriptor on gfx9 parts; a load at or past the descriptor's
 // byte count returns zeros
 constexpr int PF_RSRC_WORD3 = 0x00020000;
@@ -135,8 +138,10 @@ __global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfm
   const int nkt = (kmax + PF_KT - 1) / PF_KT;
   const int32_t* btb = bt + int64_t(b) * bt_stride;
 
-  // key group (which of every KS tiles), and thread and wave inside it
+  // key group (which of every `step` tiles), and thread and wave inside it
   const int kgrp = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(int(threadIdx.x) / (64 * NW));
+  const int step = KS == 1 || nkt < PF_SPLIT_TILES ? 1 : KS;
+  if (kgrp >= step) return;  // the barriers below are those of the waves that are left
   const int tid = threadIdx.x - kgrp * 64 * NW, wave = tid >> 6;
   uint16_t(*ks)[PF_D * PF_KT] = ks_all[kgrp];
   uint16_t(*vs)[PF_D * PF_KT] = vs_all[kgrp];
@@ -292,18 +297,18 @@ __global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfm
   // the buffer the tile read. The fetches run unconditionally (past the last tile they load
   // data no stage uses): with no branch around them, the wait for the block-table load issued
   // before a fetch counts exactly the fetch's loads instead of waiting for all of them.
-  int bt_cur = bt_of(kgrp), bt_nxt = bt_of(kgrp + KS), bt_far = bt_of(kgrp + 2 * KS);
+  int bt_cur = bt_of(kgrp), bt_nxt = bt_of(kgrp + step), bt_far = bt_of(kgrp + 2 * step);
   fetch(bt_cur);
   stage(0, kgrp);
   fetch(bt_nxt);
   __syncthreads();
-  for (int it = 0; it * KS < nkt; ++it) {
-    const int kt = it * KS + kgrp, buf = it & 1;
+  for (int it = 0; it * step < nkt; ++it) {
+    const int kt = it * step + kgrp, buf = it & 1;
     const bool real = KS == 1 || kt < nkt;  // a group past its last tile only keeps the barriers
     const int pmask = page_mask(bt_cur);
     // a tile every valid row sees whole (interior of the causal triangle, all pages valid)
     const bool full = pmask == 0xF && (kt + 1) * PF_KT <= lim_min;
-    const int bt_next_far = bt_of(kt + 3 * KS);
+    const int bt_next_far = bt_of(kt + 3 * step);
 
     // S^T for the wave's rows: 4 token blocks (one per page) x 4 d chunks, each K operand
     // serving both row blocks; d chunk outermost, so consecutive products of one accumulator
@@ -388,7 +393,7 @@ __global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfm
         }
       }
     }
-    stage(buf ^ 1, kt + KS);
+    stage(buf ^ 1, kt + step);
     fetch(bt_far);
     if (real) {
       // O += P . V over the tile's two 32-token chunks, each V operand serving both row blocks;
@@ -426,9 +431,9 @@ __global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfm
     bt_far = bt_next_far;
   }
 
-  if constexpr (KS == 2) {
+  if (KS == 2 && step == 2) {
     // group 1's sums join group 0's: [value][thread] over the tile buffers, all read by now
-    static_assert(NW == 4, "64 + 10 floats per thread of a group in the K and V buffers");
+    static_assert(KS == 1 || NW == 4, "64 + 10 floats per thread of a group in the K and V buffers");
     float* xs = reinterpret_cast<float*>(&ks_all[0][0][0]);
     float* ys = reinterpret_cast<float*>(&vs_all[0][0][0]);
     constexpr int GT = 64 * NW;
@@ -508,12 +513,16 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
   const bool wide = 2 * total_q_rows >= int64_t(wide_ppt) * num_seqs &&
                     (ceil_div(total_q_rows, wide_ppt) + num_seqs) * Hkv >= 2 * int64_t(device_cus());
   const int ppt = (wide ? 8 : 4) * PF_WROWS / G;
-  // With no more items of four waves than compute units and tables of 768 keys or more, two groups
-  // of waves share an item's keys: its chain of tiles, which is the call's time then, is half as
-  // long, for a longer start and a merge. One sequence, 32/8 heads: 300 rows behind 1500 tokens
-  // 54.2 -> 45.0 us, 40 behind 1000 35.8 -> 31.7; 300 rows on their own 17.4 against 19.3.
+  // With no more items of four waves than compute units, two groups of waves share an item's keys:
+  // its chain of tiles, which is the call's time then, is half as long, for a longer start and a
+  // merge. That pays from 8 tiles on (one sequence, 32/8 heads, 40 rows, one group against two: 7
+  // tiles 18.9 / 19.5 us, 8 20.5 / 19.8, 10 23.5 / 21.9, 12 27.0 / 24.0; 300 rows behind 1500 tokens
+  // 54.2 / 45.0). Only the tables' width is known here, so it decides the launch, and the kernel
+  // leaves shorter items under wide tables to one group where that still pays there, below 6 tiles
+  // (5: 18.0 / 17.5; 6: 17.8 / 18.7. 300 rows on their own, tables of 512 pages: 17.9 / 17.3, and
+  // 16.1 under a table of their size).
   const bool split =
-      !wide && bt_stride * PF_P >= 768 &&
+      !wide && bt_stride * PF_P >= PF_SPLIT_TABLE &&
       (ceil_div(total_q_rows, 4 * PF_WROWS / G) + num_seqs) * Hkv <= device_cus();
   // work items: at most ceil(total rows / ppt) + one partial item per sequence
   const int64_t items = (ceil_div(total_q_rows, ppt) + num_seqs) * Hkv;

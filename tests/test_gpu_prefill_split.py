@@ -90,3 +90,46 @@ def test_shared_keys_nonfinite(dev):
     dev_args[4] = torch.zeros_like(dev_args[4])   # no keys
     got = paged_attention(*dev_args[:5], cu_q=dev_args[5], q_pos_offsets=dev_args[6])
     assert bool((got == 0).all())
+
+
+@pytest.mark.parametrize("rows,ctx,Hq,Hkv,dtype", [
+    # 11, 12, 13 and 14 tiles of 64 keys: the last that one group takes, an even and an odd count
+    # for two; a last tile of one key; items of one call on either side, with the early rows of an
+    # item short of its last tiles
+    ([40], [660], 8, 8, torch.bfloat16),
+    ([40], [728], 32, 8, torch.float16),
+    ([33, 5], [736, 800], 16, 2, torch.bfloat16),
+    ([300, 20, 130], [640, 100, 702], 28, 7, torch.bfloat16),
+])
+def test_keys_shared_by_two_groups(dev, rows, ctx, Hq, Hkv, dtype):
+    args = _case(dev, rows, ctx, Hq, Hkv, dtype, 5, 50)
+    q, kp, vp, bt, kv, cu, off = (x.to(dev) for x in args)
+    got = paged_attention(q, kp, vp, bt, kv, cu_q=cu, q_pos_offsets=off).double().cpu()
+    tol = 2.0 * args[2].abs().max().item() * (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
+    assert (got - _ref(*args)).abs().max().item() <= tol
+
+
+def test_shared_keys_nonfinite_long(dev):
+    """A NaN key in either group's tiles of an item that two groups share."""
+    q, kp, vp, bt, kv, cu, off = _case(dev, [70], [900], 8, 8, torch.bfloat16, 3)
+    clean = _ref(q, kp, vp, bt, kv, cu, off)
+    kp[bt[0, 60].long(), 1, 5, 9] = math.nan      # token 969: tile 15 (group 1), the last row only
+    kp[bt[0, 32].long(), 2, 7, 0] = math.nan      # token 512: tile 8 (group 0), every row
+    got = paged_attention(*(x.to(dev) for x in (q, kp, vp, bt, kv)), cu_q=cu.to(dev),
+                          q_pos_offsets=off.to(dev)).cpu()
+    assert bool(got[69, 1].isnan().all()) and bool(got[:, 2].isnan().all())
+    keep = torch.ones(70, 8, dtype=torch.bool)
+    keep[69, 1] = keep[:, 2] = False
+    tol = 2.0 * vp.abs().max().item() * 2 ** -8
+    assert (got.double()[keep] - clean[keep]).abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("rows,ctx", [([300], [0]), ([17, 150, 301], [100, 0, 200]), ([90], [600])])
+def test_table_width_changes_nothing(dev, rows, ctx):
+    """A block table wider than its sequences need (a program with tables of one width): the same
+    bits, so the same split of the keys, which goes by the keys there are."""
+    q, kp, vp, bt, kv, cu, off = (x.to(dev) for x in _case(dev, rows, ctx, 32, 8, torch.bfloat16))
+    wide = torch.full((len(rows), 512), -1, dtype=torch.int32, device=dev)
+    wide[:, :bt.shape[1]] = bt
+    assert torch.equal(paged_attention(q, kp, vp, bt, kv, cu_q=cu, q_pos_offsets=off),
+                       paged_attention(q, kp, vp, wide, kv, cu_q=cu, q_pos_offsets=off))
