@@ -1337,14 +1337,42 @@ extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
   const int64_t a_bytes = ((ceil_div(numel, a_div) - 1) * lda + k_dim) * elt;
   const int64_t w_bytes = int64_t(n_rows) * k_dim * elt;
   // The wide kernel is built for 16-bit storage; fp32 runs the decode kernels at every size. It
-  // reads each expert's weights once where those read them once per 16 routes of it, so it takes
-  // calls of 7 or more routes per expert on average (2048 / 768 hidden / intermediate, 128
-  // experts, top-8, FFN with both GEMMs: 96 tokens 214 us against 207, 128 tokens 217 against
-  // 226, 192 tokens 225 against 243, 255 tokens 227 against 308) where the experts' tiles fill
-  // the GPU's workgroups three times over, and every call of 2048 routes.
+  // reads each expert's weights once, those once per 16 routes of it, and it has a fixed cost (the
+  // launch of its work list, the fill of its rings). So it takes over
+  //  - from the streaming kernels, which read weights as fast, where experts with more than 16
+  //    routes become common: at 9 to 14 routes per expert, sooner the larger the weights are, and
+  //    where its tiles fill the workgroups three times over (a smaller tail); rows longer than 2048
+  //    suit the streaming kernel best;
+  //  - from the others (any other K) where what they lose per byte exceeds the fixed cost: from 2
+  //    routes per expert on for large weights, like the streaming ones for small;
+  //  - with fewer tiles than workgroups, small weights, or several layers' experts in one bank (whose
+  //    average says little) at 2048 routes.
+  // Measured, bf16, decode kernel : wide kernel, us, at routes per expert (experts x rows x K):
+  //   streamed   128 x 1536 x 2048 (768 MiB, 768 tiles)  7: 121:127   9: 127:127   10: 137:127
+  //              64 x 2048 x 2048 (512, 512)             9: 83:87    10: 94:88
+  //              64 x 2048 x 1024 (256, 512)             9: 46:48    10: 51:48
+  //              64 x 2048 x 512 (128, 512)             10: 26:28    12: 29:28
+  //              128 x 768 x 512 (96, 384)              12: 23:25    14: 26:25
+  //              8 x 28672 x 4096 (1792, 896)           10: 267:296  12: 269:292  14: 336:297
+  //              128 x 3072 x 4096 (3072, 1536)         10: 460:489  12: 505:492
+  //   others     64 x 2048 x 1408 (352, 512)             2: 69:59     7: 78:62
+  //              256 x 512 x 1536 (384, 512)             2: 75:65     7: 84:68
+  //              64 x 3584 x 640 (280, 896)              4: 53:54     7: 62:55
+  //              128 x 768 x 1536 (288, 384)             4: 56:59     7: 60:59
+  //              256 x 1536 x 256 (192, 1536)            7: 42:42     9: 45:43
+  //              256 x 1024 x 256 (128, 1024)            8: 30:34    12: 36:34
+  //              128 x 512 x 512 (64, 256)               8: 15:19    14: 21:19
   const int tn = fused ? 128 : 256;  // output columns of its tiles
-  const bool many = numel >= 2048 || (numel >= 7 * int64_t(num_experts) &&
-                                      num_experts * ceil_div(out_cols, tn) >= 3 * int64_t(cus));
+  const int64_t tiles = num_experts * ceil_div(out_cols, tn), mib = num_experts * w_bytes >> 20;
+  const bool streamed = fused || k_dim > EG_COLS_MAX_K
+                            ? k_dim % 1024 == 0 && k_dim <= 4096
+                            : k_dim == 512 || k_dim == 768 || k_dim == 1024;
+  const int line = mib < 140  ? 14
+                   : !streamed ? (mib < 256 ? 8 : mib < 340 ? 7 : 2)
+                   : mib < 256 || k_dim > 2048 ? 12
+                   : tiles < 3 * int64_t(cus)  ? 10
+                                               : 9;
+  const bool many = numel >= 2048 || (numel >= line * int64_t(num_experts) && tiles >= cus && mib >= 64);
   if (!f32 && many && a_bytes < (int64_t(1) << 31) && w_bytes < (int64_t(1) << 31) &&
       max_num_tokens_padded < (int64_t(1) << 29) &&
       numel < (int64_t(1) << 29)) {

@@ -157,3 +157,42 @@ def test_ffn_fewer_second_matrices(dev, T):
     held = (ids >= 0) & (ids < E2)
     err = (part[held].float() - full[held].float()).abs().max()
     assert err <= 2.0 ** -7 * full[held].float().abs().max()   # one rounding step: other sum order
+
+
+@pytest.mark.parametrize("E,n_rows,K,activation,line", [
+    (32, 2 * 3072, 1000, "silu", 2), (64, 2304, 1408, None, 2),    # no streaming kernel for this K
+    (64, 2048, 1104, None, 7), (64, 2048, 1000, None, 8), (64, 2 * 2048, 264, "silu", 14),
+    (128, 2048, 768, None, 9), (64, 2 * 1024, 2048, "gelu_tanh", 10),   # one for this
+    (64, 3072, 512, None, 12), (32, 2 * 1024, 3072, "silu", 12), (64, 2 * 512, 1024, "gelu", 14),
+])
+def test_either_side_of_the_line(dev, E, n_rows, K, activation, line):
+    """Calls of one route fewer and of as many as the wide kernel takes."""
+    g = torch.Generator(device=dev).manual_seed(K)
+    w = (torch.randn(E, n_rows, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    for numel in (line * E - 1, line * E):
+        a = torch.randn(numel, K, generator=g, device=dev).to(torch.bfloat16)
+        ids = torch.randint(0, E, (numel, 1), generator=g, device=dev, dtype=torch.int32)
+        s, e, npp = moe_align_block_size(ids, 16, E)
+        got = moe_expert_gemm(a, w, None, s, e, npp, 16, numel, 1, activation=activation)
+        ref = torch.empty(numel, n_rows, device=dev)
+        for x in range(E):
+            at = (ids.view(-1) == x).nonzero().view(-1)
+            ref[at] = a[at].float() @ w[x].float().t()
+        bound = 0.0
+        if activation:
+            gate, up = ref.to(torch.bfloat16).float().chunk(2, -1)
+
+            def f(x):
+                return torch.nn.functional.silu(x) if activation == "silu" else \
+                    torch.nn.functional.gelu(x, approximate="tanh" if activation == "gelu_tanh"
+                                             else "none")
+
+            # a first sum on the other side of a rounding point: one step (2^-7) of the gate or of up
+            step = torch.maximum((f(gate * (1 + 2 ** -7)) - f(gate)).abs(),
+                                 (f(gate * (1 - 2 ** -7)) - f(gate)).abs())
+            ref = f(gate) * up
+            bound = step * up.abs() * (1 + 2 ** -7) + ref.abs() * 2 ** -7
+        diff = (got.float() - ref).abs()
+        # one step of the result's own, and fp32 sums of K products in another order (2^-20 of ~K^0.5)
+        assert bool((diff <= bound + ref.abs() * 2 ** -7 + 2 ** -20 * K ** 0.5).all()), numel
+        assert (got != ref.to(torch.bfloat16)).float().mean().item() < 0.01, numel
