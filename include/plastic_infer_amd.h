@@ -364,6 +364,15 @@ int pia_moe_ffn(void* out, void* route_out, const void* x, int64_t ldx, const vo
                 int activation, int weight_on_input, int dtype, void* act, int64_t ld_act,
                 void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The same over banks that hold more experts than a call's ids come from: w1 and w2 have
+ * num_experts slots (those of several layers, say), ids are slots, and layer_experts is the number
+ * of a layer's experts (0: not said, as pia_moe_ffn). Only the kernels' tile sizes go by it. */
+int pia_moe_ffn_bank(void* out, void* route_out, const void* x, int64_t ldx, const void* w1,
+                     const void* w2, const float* topk_weights, const int32_t* topk_ids,
+                     int64_t num_tokens, int topk, int num_experts, int layer_experts, int hidden,
+                     int inter, int activation, int weight_on_input, int dtype, void* act,
+                     int64_t ld_act, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* out = s / sqrt(mean(s^2) + eps) * weight over rows of n elements, s = x, or x + residual rounded
  * to the dtype and written to sum (a buffer of its own) when residual is given. The
  * reference's rms_norm (src/plastic_infer/exec/attention.py:77-79) with fp32 arithmetic and one

@@ -1289,13 +1289,14 @@ extern "C" int64_t pia_moe_expert_gemm_workspace_bytes(int64_t max_num_tokens_pa
   return (2 * ceil_div(max_num_tokens_padded, block_m) + 2 + TG_XCDS) * int64_t(sizeof(int32_t));
 }
 
-extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
-                                   const float* topk_weights, const int32_t* sorted_token_ids,
-                                   const int32_t* expert_ids, const int32_t* num_tokens_post_pad,
-                                   int64_t max_num_tokens_padded, int block_m, int64_t numel,
-                                   int a_div, int64_t lda, int num_experts, int n_rows, int k_dim,
-                                   int64_t ldo, int activation, int mul_routed_weight, int dtype,
-                                   void* workspace, int64_t workspace_bytes, void* stream) {
+namespace pia {
+
+int expert_gemm(void* out, const void* a, const void* w, const float* topk_weights,
+                const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                const int32_t* num_tokens_post_pad, int64_t max_num_tokens_padded, int block_m,
+                int64_t numel, int a_div, int64_t lda, int num_experts, int layer_experts,
+                int n_rows, int k_dim, int64_t ldo, int activation, int mul_routed_weight,
+                int dtype, void* workspace, int64_t workspace_bytes, void* stream) {
   if (dtype != PIA_DTYPE_BF16 && dtype != PIA_DTYPE_F16 && dtype != PIA_DTYPE_F32)
     return fail(PIA_EUNSUPPORTED, "moe_expert_gemm: dtype must be bf16, fp16 or fp32");
   if (activation < PIA_ACT_NONE || activation > PIA_ACT_GELU_TANH)
@@ -1363,7 +1364,9 @@ extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
   //              256 x 1024 x 256 (128, 1024)            8: 30:34    12: 36:34
   //              128 x 512 x 512 (64, 256)               8: 15:19    14: 21:19
   const int tn = fused ? 128 : 256;  // output columns of its tiles
-  const int64_t tiles = num_experts * ceil_div(out_cols, tn), mib = num_experts * w_bytes >> 20;
+  layer_experts = std::min(layer_experts, num_experts);
+  const int64_t layer = layer_experts > 0 ? layer_experts : num_experts;
+  const int64_t tiles = layer * ceil_div(out_cols, tn), mib = layer * w_bytes >> 20;
   const bool streamed = fused || k_dim > EG_COLS_MAX_K
                             ? k_dim % 1024 == 0 && k_dim <= 4096
                             : k_dim == 512 || k_dim == 768 || k_dim == 1024;
@@ -1372,7 +1375,7 @@ extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
                    : mib < 256 || k_dim > 2048 ? 12
                    : tiles < 3 * int64_t(cus)  ? 10
                                                : 9;
-  const bool many = numel >= 2048 || (numel >= line * int64_t(num_experts) && tiles >= cus && mib >= 64);
+  const bool many = numel >= 2048 || (numel >= line * layer && tiles >= cus && mib >= 64);
   if (!f32 && many && a_bytes < (int64_t(1) << 31) && w_bytes < (int64_t(1) << 31) &&
       max_num_tokens_padded < (int64_t(1) << 29) &&
       numel < (int64_t(1) << 29)) {
@@ -1382,11 +1385,15 @@ extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
     int32_t* seg_xstart = seg_count + 1;                             // [max_blocks]
     int32_t* xcd_items = seg_xstart + max_blocks;                   // [8]
     // Row tile: the plan rows of an expert at the call's mean plus two deviations of a random
-    // routing. A bank of more than 256 slots holds several layers' experts, of which a call
-    // routes to one layer's: taken as 128. (FFN, 128 experts top-8: 333 tokens 237 us at RF 1
-    // against 306 at the former 320 rows for every call, 1024 tokens 265 at RF 2 against 372,
-    // 2048 tokens 310 at RF 3 against 388.)
-    const double mean = double(numel) / (num_experts <= 256 ? num_experts : 128);
+    // routing, over the experts of a layer, which only the caller knows where w is a bank of slots
+    // (layer_experts). Not told, up to 256 are taken as one layer's and more as a bank of layers of
+    // 128. What a wrong guess costs (FFN, 2048 / 768 hidden / intermediate, top-8, 256 slots, 3000
+    // tokens): 256 experts taken as 128 604 us against 516, 128 taken as 256 493 against 367. It
+    // goes by the call's sizes alone, so that the parts of a split call take the same tiles. (FFN,
+    // 128 experts top-8: 333 tokens 237 us at RF 1 against 306 at 320 rows for every call, 1024
+    // tokens 265 at RF 2 against 372, 2048 tokens 310 at RF 3 against 388.)
+    const int experts = layer_experts > 0 ? layer_experts : num_experts <= 256 ? num_experts : 128;
+    const double mean = double(numel) / experts;
     const double want = mean + 2.0 * std::sqrt(mean);
     const int rf = want <= 64 ? 1 : want <= 128 ? 2 : want <= 192 ? 3 : 5;
     const int bm = 64 * rf;
@@ -1551,6 +1558,21 @@ extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
 #undef PIA_EG
 #undef PIA_EG_K
   return check_launch(cols ? "moe_gemm_cols" : "moe_gemm_splitk");
+}
+
+}  // namespace pia
+
+extern "C" int pia_moe_expert_gemm(void* out, const void* a, const void* w,
+                                   const float* topk_weights, const int32_t* sorted_token_ids,
+                                   const int32_t* expert_ids, const int32_t* num_tokens_post_pad,
+                                   int64_t max_num_tokens_padded, int block_m, int64_t numel,
+                                   int a_div, int64_t lda, int num_experts, int n_rows, int k_dim,
+                                   int64_t ldo, int activation, int mul_routed_weight, int dtype,
+                                   void* workspace, int64_t workspace_bytes, void* stream) {
+  return expert_gemm(out, a, w, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad,
+                     max_num_tokens_padded, block_m, numel, a_div, lda, num_experts, 0, n_rows,
+                     k_dim, ldo, activation, mul_routed_weight, dtype, workspace, workspace_bytes,
+                     stream);
 }
 
 extern "C" int pia_act_and_mul(void* out, const void* x, int64_t rows, int64_t d, int activation,

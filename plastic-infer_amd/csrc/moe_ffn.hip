@@ -63,7 +63,20 @@ extern "C" int pia_moe_ffn(void* out, void* route_out, const void* x, int64_t ld
                            int activation, int weight_on_input, int dtype, void* act,
                            int64_t ld_act, void* workspace, int64_t workspace_bytes,
                            void* stream) {
-  if (num_tokens < 0 || topk <= 0 || num_experts <= 0 || hidden <= 0 || inter <= 0)
+  return pia_moe_ffn_bank(out, route_out, x, ldx, w1, w2, topk_weights, topk_ids, num_tokens, topk,
+                          num_experts, 0, hidden, inter, activation, weight_on_input, dtype, act,
+                          ld_act, workspace, workspace_bytes, stream);
+}
+
+extern "C" int pia_moe_ffn_bank(void* out, void* route_out, const void* x, int64_t ldx,
+                                const void* w1, const void* w2, const float* topk_weights,
+                                const int32_t* topk_ids, int64_t num_tokens, int topk,
+                                int num_experts, int layer_experts, int hidden, int inter,
+                                int activation, int weight_on_input, int dtype, void* act,
+                                int64_t ld_act, void* workspace, int64_t workspace_bytes,
+                                void* stream) {
+  if (num_tokens < 0 || topk <= 0 || num_experts <= 0 || layer_experts < 0 || hidden <= 0 ||
+      inter <= 0)
     return fail(PIA_EINVAL, "moe_ffn: invalid size");
   if (dtype != PIA_DTYPE_BF16 && dtype != PIA_DTYPE_F16 && dtype != PIA_DTYPE_F32)
     return fail(PIA_EUNSUPPORTED, "moe_ffn: dtype must be bf16, fp16 or fp32");
@@ -88,15 +101,14 @@ extern "C" int pia_moe_ffn(void* out, void* route_out, const void* x, int64_t ld
                                         num_experts, FFN_BLOCK, o.mpad, ws + o.align_ws,
                                         o.align_bytes, stream))
     return rc;
-  if (int rc = pia_moe_expert_gemm(a, x, w1, topk_weights, sorted, experts, npp, o.mpad, FFN_BLOCK,
-                                   o.numel, topk, ldx, num_experts, 2 * inter, hidden, lda,
-                                   activation, weight_on_input ? 1 : 0, dtype, ws + o.gemm_ws,
-                                   o.gemm_bytes, stream))
+  if (int rc = expert_gemm(a, x, w1, topk_weights, sorted, experts, npp, o.mpad, FFN_BLOCK,
+                           o.numel, topk, ldx, num_experts, layer_experts, 2 * inter, hidden, lda,
+                           activation, weight_on_input ? 1 : 0, dtype, ws + o.gemm_ws,
+                           o.gemm_bytes, stream))
     return rc;
-  if (int rc = pia_moe_expert_gemm(r, a, w2, topk_weights, sorted, experts, npp, o.mpad, FFN_BLOCK,
-                                   o.numel, 1, lda, num_experts, hidden, inter, hidden,
-                                   PIA_ACT_NONE, weight_on_input ? 0 : 1, dtype, ws + o.gemm_ws,
-                                   o.gemm_bytes, stream))
+  if (int rc = expert_gemm(r, a, w2, topk_weights, sorted, experts, npp, o.mpad, FFN_BLOCK, o.numel,
+                           1, lda, num_experts, layer_experts, hidden, inter, hidden, PIA_ACT_NONE,
+                           weight_on_input ? 0 : 1, dtype, ws + o.gemm_ws, o.gemm_bytes, stream))
     return rc;
   if (!out) return 0;
   return pia_moe_sum_reduce(out, r, num_tokens, topk, hidden, dtype, stream);

@@ -57,6 +57,15 @@ int launch_rows(int dtype, void* out, const void* q, const void* k_pages, const 
                 int Hq, int Hkv, int D, int P, int64_t num_pages, float scale_log2,
                 hipStream_t s);
 
+// pia_moe_expert_gemm with the number of experts that a layer's ids come from, where w holds more
+// slots than that (0: not said).
+int expert_gemm(void* out, const void* a, const void* w, const float* topk_weights,
+                const int32_t* sorted_token_ids, const int32_t* expert_ids,
+                const int32_t* num_tokens_post_pad, int64_t max_num_tokens_padded, int block_m,
+                int64_t numel, int a_div, int64_t lda, int num_experts, int layer_experts,
+                int n_rows, int k_dim, int64_t ldo, int activation, int mul_routed_weight,
+                int dtype, void* workspace, int64_t workspace_bytes, void* stream);
+
 // ---------------------------------------------------------------------------------------------
 // Device helpers
 // ---------------------------------------------------------------------------------------------

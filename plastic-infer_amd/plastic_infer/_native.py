@@ -58,6 +58,8 @@ _SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "pia_moe_ffn_workspace_bytes": (_L, [_L, _I, _I, _I, _I, _I, _I, _I]),
     "pia_moe_ffn": (_I, [_P, _P, _P, _L, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _I, _P, _L,
                          _P, _L, _P]),
+    "pia_moe_ffn_bank": (_I, [_P, _P, _P, _L, _P, _P, _P, _P, _L, _I, _I, _I, _I, _I, _I, _I, _I,
+                              _P, _L, _P, _L, _P]),
     "pia_rms_norm": (_I, [_P, _P, _P, _P, _P, _L, _I, _F, _I, _P]),
     "pia_qk_norm_rope": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _L, _I, _I, _I, _F, _I, _P]),
     "pia_moe_sum_reduce": (_I, [_P, _P, _L, _I, _I, _I, _P]),

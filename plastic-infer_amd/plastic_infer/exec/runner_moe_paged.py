@@ -184,7 +184,8 @@ class MoePagedDecoder:
             slots = topk_ids.clone()
             self.cache.ensure_experts(layer, slots)
             self.cache.copy_missing()
-            return fused_experts_decode_impl(h, gate_up, down, topk_w, slots), {"slots": slots}
+            return fused_experts_decode_impl(h, gate_up, down, topk_w, slots,
+                                             layer_experts=self.cfg.n_experts), {"slots": slots}
         routes = self.cache.stage_layer(layer, topk_ids)
         B, k = topk_ids.shape
         route_out = torch.empty(B, k, h.shape[1], dtype=h.dtype, device=h.device)
@@ -194,13 +195,15 @@ class MoePagedDecoder:
         if routes.issued is not None:
             ev["a0"] = torch.cuda.Event(enable_timing=True)
             ev["a0"].record(compute)
-        routed_ffn_routes(h, gate_up, down, topk_w, routes.in_hbm, route_out, act_buffer=act)
+        routed_ffn_routes(h, gate_up, down, topk_w, routes.in_hbm, route_out, act_buffer=act,
+                          layer_experts=self.cfg.n_experts)
         if routes.issued is not None:
             ev["a1"] = torch.cuda.Event(enable_timing=True)
             ev["a1"].record(compute)
         compute.wait_event(routes.ready)
         if routes.copied_experts:   # else every route was in the first group
-            routed_ffn_routes(h, gate_up, down, topk_w, routes.copied, route_out, act_buffer=act)
+            routed_ffn_routes(h, gate_up, down, topk_w, routes.copied, route_out, act_buffer=act,
+                              layer_experts=self.cfg.n_experts)
         out = torch.empty_like(h)
         moe_sum_reduce(route_out, out)
         info = {"routes": routes, "events": ev}

@@ -74,13 +74,16 @@ def routed_ffn_routes(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
                       topk_weights: torch.Tensor, topk_ids: torch.Tensor,
                       route_out: torch.Tensor, activation: str = "silu",
                       apply_router_weight_on_input: bool = False,
-                      act_buffer: torch.Tensor | None = None) -> torch.Tensor:
+                      act_buffer: torch.Tensor | None = None,
+                      layer_experts: int | None = None) -> torch.Tensor:
     """The routed FFN of every route whose id is in [0, E), into route_out [T, k, H]: row
     (t, s) = w2[id] . act(w1[id] . x_t) times the routing weight, rounded to the storage dtype
     at the reference's points. Routes with id -1 are left untouched, so the routes of one
     token can be computed in several calls (e.g. experts already in HBM first, copied ones
     after their copies land) and summed once with moe_sum_reduce: the result is bit-identical
-    to one call over all routes. act_buffer [T * k, I] may be shared between such calls."""
+    to one call over all routes. act_buffer [T * k, I] may be shared between such calls.
+    layer_experts: how many experts a layer has, where w1 and w2 are banks of more slots than that
+    (the kernels' tiles are sized by it; such calls give the same one)."""
     M, H = hidden_states.shape
     E, two_i, _ = w1.shape
     k = topk_ids.shape[1]
@@ -115,13 +118,13 @@ def routed_ffn_routes(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
         route_out.masked_fill_((ids >= E2) & (ids <= E), 0)
         w1 = w1[:E2]
     _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, apply_router_weight_on_input,
-         None, route_out, act_buffer)
+         None, route_out, act_buffer, layer_experts)
     return route_out
 
 
 def _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, on_input, out, route_out=None,
-         act_buffer=None) -> None:
-    """The FFN of arguments already checked (pia_moe_ffn), every buffer not given in one
+         act_buffer=None, layer_experts=None) -> None:
+    """The FFN of arguments already checked (pia_moe_ffn_bank), every buffer not given in one
     workspace."""
     act = ACTIVATION_CODES.get(activation)
     if act is None:
@@ -134,45 +137,50 @@ def _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, on_input, ou
     ws_bytes = N.query("pia_moe_ffn_workspace_bytes", M, k, E, H, inter, dt,
                        1 if act_buffer is None else 0, 1 if route_out is None else 0)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    N.call("pia_moe_ffn", N.ptr(out), N.ptr(route_out), hidden_states.data_ptr(),
+    N.call("pia_moe_ffn_bank", N.ptr(out), N.ptr(route_out), hidden_states.data_ptr(),
            hidden_states.stride(0), w1.data_ptr(), w2.data_ptr(), weights.data_ptr(),
-           ids.data_ptr(), M, k, E, H, inter, act, 1 if on_input else 0, dt, N.ptr(act_buffer),
+           ids.data_ptr(), M, k, E, layer_experts or 0, H, inter, act, 1 if on_input else 0, dt, N.ptr(act_buffer),
            0 if act_buffer is None else act_buffer.stride(0), ws.data_ptr(), ws_bytes,
            N.stream_of(dev))
 
 
 def _routed_ffn(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
                 topk_weights: torch.Tensor, topk_ids: torch.Tensor, activation: str,
-                apply_router_weight_on_input: bool, out: torch.Tensor) -> torch.Tensor:
+                apply_router_weight_on_input: bool, out: torch.Tensor,
+                layer_experts: int | None) -> torch.Tensor:
     if topk_ids.numel():
         _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation,
-             apply_router_weight_on_input, out)
+             apply_router_weight_on_input, out, layer_experts=layer_experts)
     return out
 
 
 def fused_experts_impl(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
                        topk_weights: torch.Tensor, topk_ids: torch.Tensor,
                        activation: str = "silu",
-                       apply_router_weight_on_input: bool = False) -> torch.Tensor:
+                       apply_router_weight_on_input: bool = False,
+                       layer_experts: int | None = None) -> torch.Tensor:
     """Returns ``hidden_states`` itself, overwritten with the routed output (the reference's
     contract: a caller that still needs the input must read it first or pass a copy).
-    w1 [E, 2I, H] (gate rows then up rows), w2 [E, H, I]; ids in [0, E)."""
+    w1 [E, 2I, H] (gate rows then up rows), w2 [E, H, I]; ids in [0, E). layer_experts as for
+    routed_ffn_routes."""
     _check_ffn_args(hidden_states, w1, w2, topk_weights, topk_ids, activation)
     return _routed_ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation,
-                       apply_router_weight_on_input, hidden_states)
+                       apply_router_weight_on_input, hidden_states, layer_experts)
 
 
 def fused_experts_decode_impl(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
                               topk_weights: torch.Tensor, topk_ids: torch.Tensor,
                               activation: str = "silu",
-                              apply_router_weight_on_input: bool = False) -> torch.Tensor:
-    """The routed FFN into a new tensor (ids are expert or slot indices into w1 / w2)."""
+                              apply_router_weight_on_input: bool = False,
+                              layer_experts: int | None = None) -> torch.Tensor:
+    """The routed FFN into a new tensor (ids are expert or slot indices into w1 / w2).
+    layer_experts as for routed_ffn_routes."""
     _check_ffn_args(hidden_states, w1, w2, topk_weights, topk_ids, activation)
     assert topk_weights.dtype == torch.float32
     assert topk_ids.dtype == torch.int32
     out = torch.empty_like(hidden_states)
     return _routed_ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation,
-                       apply_router_weight_on_input, out)
+                       apply_router_weight_on_input, out, layer_experts)
 
 
 class FusedMoe(BaseMoeBackend):
@@ -184,7 +192,8 @@ class FusedMoe(BaseMoeBackend):
                                             gating_output=gating_output, topk=topk,
                                             renormalize=renormalize)
         return fused_experts_impl(hidden_states, w1, w2, topk_weights, topk_ids, activation,
-                                  apply_router_weight_on_input=apply_router_weight_on_input)
+                                  apply_router_weight_on_input=apply_router_weight_on_input,
+                                  layer_experts=gating_output.shape[1])
 
 
 __all__ = ["fused_topk", "moe_align_block_size", "fused_experts_impl",

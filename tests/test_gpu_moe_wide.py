@@ -11,6 +11,7 @@ import torch
 import oracle.fused_experts as OF
 import oracle.moe_route as OM
 from plastic_infer.kernel import moe_align_block_size, moe_expert_gemm
+from plastic_infer.kernel.moe_ops import moe_sum_reduce
 from plastic_infer.moe.fused import (
     fused_experts_decode_impl, fused_experts_impl, routed_ffn_routes)
 
@@ -196,3 +197,25 @@ def test_either_side_of_the_line(dev, E, n_rows, K, activation, line):
         # one step of the result's own, and fp32 sums of K products in another order (2^-20 of ~K^0.5)
         assert bool((diff <= bound + ref.abs() * 2 ** -7 + 2 ** -20 * K ** 0.5).all()), numel
         assert (got != ref.to(torch.bfloat16)).float().mean().item() < 0.01, numel
+
+
+@pytest.mark.parametrize("T", [40, 1100])
+def test_bank_of_several_layers(dev, T):
+    """One layer's experts among the slots of a larger bank: the same results with and without the
+    number of a layer's experts, whole or in the two parts of a split call."""
+    E, used, k, H, I = 256, 32, 4, 128, 96
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    w1 = (torch.randn(E, 2 * I, H, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    w2 = (torch.randn(E, H, I, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    tw = torch.rand(T, k, generator=g).to(dev)
+    ids = torch.randint(100, 100 + used, (T, k), generator=g).to(torch.int32).to(dev)
+    plain = fused_experts_decode_impl(x, w1, w2, tw, ids)
+    told = fused_experts_decode_impl(x, w1, w2, tw, ids, layer_experts=used)
+    _mostly_equal(told, plain, "layer_experts")
+    rows = torch.empty(T, k, H, dtype=torch.bfloat16, device=dev)
+    for part in (ids < 110, ids >= 110):
+        routed_ffn_routes(x, w1, w2, tw, torch.where(part, ids, -1), rows, layer_experts=used)
+    out = torch.empty_like(x)
+    moe_sum_reduce(rows, out)
+    assert torch.equal(out, told)
