@@ -19,13 +19,13 @@ EPS = 1e-5   # of the reference's rms_norm
 def _fits(*tensors: torch.Tensor) -> bool:
     """Contiguous device tensors of one dtype that the kernels are built for, with no derivative
     to be taken of them in either mode (inside a dual level any of them may carry a tangent)."""
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors) \
-            or getattr(forward_ad, "_current_level", -1) >= 0:
+    if getattr(forward_ad, "_current_level", -1) >= 0:
         return False
-    dt = tensors[0].dtype
-    return dt in (torch.bfloat16, torch.float16, torch.float32) and all(
-        t.dtype == dt and t.is_contiguous() and t.device == tensors[0].device for t in tensors) \
-        and tensors[0].device.type == "cuda"
+    dt, dev, grad = tensors[0].dtype, tensors[0].device, torch.is_grad_enabled()
+    for t in tensors:
+        if t.dtype != dt or not t.is_contiguous() or t.device != dev or (grad and t.requires_grad):
+            return False
+    return dev.type == "cuda" and dt in (torch.bfloat16, torch.float16, torch.float32)
 
 
 def _plain(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
