@@ -18,7 +18,7 @@ reference torch path on this host's cores, on a bounded sample of the same input
   python bench.py [--steps K] [--warmup W] [--gpus 1] [--cpu-sample-seqs S] [--no-cpu-baseline]
                   [--separate-write] [--dtype bf16|fp16|fp32]
                   # fp16: the same step on fp16 pools (the same kernel); fp32: on fp32 pools,
-                  # which the general tiled kernel serves (write and attention as two calls)
+                  # which the fp32-precision kernel serves (write and attention as two calls)
   python bench.py --calibrate-copy     # 1 GiB read + 1 GiB write elementwise copy, three times:
                                        # the known-size reference for HBM byte counters
   python bench.py --workload decode-gqa8     # Qwen3-30B-A3B attention layer: 64 x 4096 tokens,
@@ -65,7 +65,7 @@ MAX_PAGES = LEN_HI // P
 WORKLOAD = "qwen3-8b paged decode: kv scatter + gqa paged attention, 1 layer"
 PMC_FILE = ROOT / "profiles" / "paged_decode_qwen3_8b_b256_pmc.json"
 PMC_FP16_FILE = ROOT / "profiles" / "paged_decode_qwen3_8b_b256_fp16_pmc.json"
-PMC_FP32_FILE = ROOT / "profiles" / "paged_attention_tiled_qwen3_8b_b256_fp32_pmc.json"
+PMC_FP32_FILE = ROOT / "profiles" / "paged_decode_f32_qwen3_8b_b256_pmc.json"
 GQA8_PMC_FILE = ROOT / "profiles" / "paged_decode_gqa8_qwen3_30b_b64_pmc.json"
 
 
@@ -1570,7 +1570,7 @@ def main() -> int:
                     help="decode: write the new rows with kv_scatter, then attend (two calls)")
     ap.add_argument("--dtype", choices=("bf16", "fp16", "fp32"), default="bf16",
                     help="decode: storage dtype of the pools, q and the new rows (fp32: the "
-                         "general tiled kernel, write and attention as two calls)")
+                         "fp32-precision kernel, write and attention as two calls)")
     ap.add_argument("--workload", choices=("decode", "decode-gqa8", "prefill-write",
                                            "moe-permute", "expert-stream", "moe-experts",
                                            "moe-experts-prefill", "prefill-stream", "kv-sink",
@@ -1699,8 +1699,8 @@ def main() -> int:
         "step": "kv_scatter + paged_decode_attention" if separate
                 else "paged_decode_append_attention (write + attention, one call)",
         "roofline": {
-            "kernel": ("paged_attention_tiled<fp32, 32-key chunks, 16-byte loads> "
-                       "(one attention call)" if args.dtype == "fp32" else
+            "kernel": ("paged_decode_f32<fp32, 128> (one attention call)"
+                       if args.dtype == "fp32" else
                        f"paged_decode_stream<4, {args.dtype}> (one attention call)"
                        if separate else f"paged_decode_stream<4, append, {args.dtype}> "
                        "(one write + attention launch)"),
