@@ -173,9 +173,10 @@ int pia_paged_decode_attention(void* out, const void* q, int64_t q_seq_stride,
  * pia_paged_decode_attention gives over the updated pools (same arguments, workspace and
  * rules). A row whose L_b is 0 or exceeds bt_stride * page_size writes no slot; a slot whose
  * page id is outside [0, num_pages) is not written and the new token is then no key.
- * The fast kernel (the same shapes as pia_paged_decode_attention's) takes the new token's K / V
- * from k_new / v_new and stores them into the slot itself, so the step has no separate write
- * launch ahead of the attention; other shapes write the slots with a small kernel first.
+ * The kernels that split the batch over persistent waves (the fast one, and for the other shapes
+ * the one that needs pia_paged_decode_split_scratch_bytes) take the new token's K / V from k_new /
+ * v_new and store them into the slot themselves, so the step has no separate write launch ahead of
+ * the attention; the general kernel's calls write the slots with a small kernel first.
  * A slot must belong to one row only (a row's new-token page is not read by another row of the
  * call), as with any slot that a decode step writes.
  * ------------------------------------------------------------------------------------------- */
@@ -351,8 +352,8 @@ int pia_moe_sum_reduce(void* out, const void* in, int64_t num_tokens, int topk, 
  * src/plastic_infer/moe/fused.py:276-359) as one call: pia_moe_align_block_size (blocks of 16),
  * pia_moe_expert_gemm over w1 [E, 2 inter, hidden] with the activation, then over w2
  * [E, hidden, inter], and pia_moe_sum_reduce into out [T, hidden]. x is [T, hidden] with row stride
- * ldx. route_out [T, topk, hidden]: the routes' rows before the sum (rows of ids outside [0, E)
- * are left as they are); NULL: kept in the workspace. out may be NULL when route_out is given (no
+ * ldx. route_out [T, topk, hidden]: the routes' rows before the sum (those of id E are zeros, those
+ * of ids outside [0, E] are left as they are); NULL: kept in the workspace. out may be NULL when route_out is given (no
  * sum), and may be x. act [T * topk, inter] with row stride ld_act, or NULL: kept in the workspace.
  * workspace: 256-byte aligned, of pia_moe_ffn_workspace_bytes (own_act / own_route: whether act /
  * route_out are NULL). */
@@ -406,10 +407,11 @@ int pia_qk_norm_rope(void* q_out, void* k_out, const void* q, const void* k, con
  * bf16, fp16 or fp32 (dtype; for fp32 round() is the identity and the products are fp32
  * MFMA products), topk_weights fp32 [numel]. k_dim and lda multiples of 8 (bf16 / fp16) or 4
  * (fp32); a and w 16-byte aligned; block_m a multiple of 16; a holds ceil(numel / a_div) rows.
- * Small calls (decode: fewer than 2048 routes) and every fp32 call run a split-K kernel over
- * 16-row plan blocks that streams each expert's W once per block; larger bf16 / fp16 calls run
- * an LDS-tiled kernel over the experts present in the plan (tiles of up to 320 routes x 256 W
- * rows, so that each expert's W is streamed once when it serves up to 320 routes). The first
+ * Every fp32 call and bf16 / fp16 calls of few routes per expert run kernels over 16-row plan
+ * blocks that stream each expert's W once per block; bf16 / fp16 calls of 2 to 14 routes per expert
+ * and more (by K and the size of the weights), and all of 2048 routes, run an LDS-tiled kernel over
+ * the experts present in the plan (tiles of 64 to 320 routes x 256 W rows, so that each expert's W
+ * is streamed once when its routes fit one). The choice goes by sizes, never by the plan. The first
  * GEMM of the FFN is a_div = top_k
  * (a = hidden [T, H]) with the activation; the second is a_div = 1 (a = the first GEMM's
  * output [T*k, I]) without it, ldo = H, writing [T, k, H] for pia_moe_sum_reduce.

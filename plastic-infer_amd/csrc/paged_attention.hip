@@ -1462,8 +1462,9 @@ __global__ __launch_bounds__(64, 1) void paged_decode_mfma(
 // Block-table entries are fetched two steps ahead, before the step's tile loads: vector memory
 // counters retire in order, so a wait on them then holds for no tile load behind them.
 // Measured against paged_attention_tiled, which served these shapes (whole calls with the KV
-// append): 32 sequences of 1..2048 tokens, 16/8 heads of 128, fp32: 358.4 -> 59.7 us (4.4 TB/s); 48 of
-// 256..4096, 32/8 heads of 64, bf16: 471.0 -> 55.6 us (4.1 TB/s).
+// append): 32 sequences of 1..2048 tokens, 16/8 heads of 128, fp32: 358 -> 58.1 us (4.5 TB/s); 48 of
+// 256..4096, 32/8 heads of 64, bf16: 471 -> 54.2 us (4.2 TB/s); 256 of 512..8192, 32/8 heads of 128,
+// fp32, no append: 3283 -> 1397 us (6.5 TB/s).
 // ---------------------------------------------------------------------------------------------
 template <int DT, int D, bool APPEND>
 __global__ __launch_bounds__(64, 2) void paged_decode_f32(

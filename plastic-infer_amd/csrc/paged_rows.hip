@@ -23,8 +23,8 @@
 // Measured against paged_attention_tiled, which ran a workgroup per row: 2 sequences of 300..600
 // rows behind 0..512 tokens, 16/8 heads of 128, fp32:
 // 743 -> 116 us, 98 us with the heads dealt to the XCDs, 93 us with the K loads' lanes in the order
-// of their vectors (8 sequences of 1024 rows behind 3072, 28/4 heads, bf16: 1964 -> 1504 us), 83 us
-// with the sums in pairs (attn_tiles_f32.h). Two
+// of their vectors (8 sequences of 1024 rows behind 3072, 28/4 heads, bf16: 23.3 ms, 1964, then 1504
+// us), 83 us with the sums in pairs (attn_tiles_f32.h). Two
 // 16-row blocks per wave, which halve the tile reads: 88 and 1535 us, and 28.6 against 23.0 us for
 // 2 short ones at head_dim 64; not kept.
 #include <algorithm>

@@ -50,7 +50,8 @@ def _ref(q, kp, vp, bt, kv, cu, ctx):
     return out
 
 
-@pytest.mark.parametrize("width", [0, 50])   # 50 pages: with few items, keys shared by two groups
+# 50 pages: the launch of two wave groups where items are few, which share keys from six tiles on
+@pytest.mark.parametrize("width", [0, 50])
 @pytest.mark.parametrize("rows,ctx,Hq,Hkv,dtype", [
     # few items: one tile, an odd count of tiles, a group without a tile for the first rows,
     # ragged sequences; kv heads that do and do not divide over the XCDs
@@ -73,13 +74,13 @@ def test_prefill_shapes(dev, rows, ctx, Hq, Hkv, dtype, width):
 
 
 def test_shared_keys_nonfinite(dev):
-    """A NaN or infinite key or value reaches the rows that see it, in either group's tiles, and no
-    other row; a row with no key at all is zero."""
+    """A NaN or infinite key or value reaches the rows that see it and no other row; a row with no key
+    at all is zero. In the launch of two wave groups, an item of three tiles (one group's)."""
     rows, ctx, Hq, Hkv = [70], [100], 8, 8
     q, kp, vp, bt, kv, cu, off = _case(dev, rows, ctx, Hq, Hkv, torch.bfloat16, 3, 50)
     clean = _ref(q, kp, vp, bt, kv, cu, off)
-    kp[bt[0, 10].long(), 1, 5, 9] = math.nan      # token 169: tile 2 (group 0), the last row only
-    kp[bt[0, 4].long(), 2, 7, 0] = math.nan       # token 64: tile 1 (group 1), every row
+    kp[bt[0, 10].long(), 1, 5, 9] = math.nan      # token 169: tile 2, the last row only
+    kp[bt[0, 4].long(), 2, 7, 0] = math.nan       # token 64: tile 1, every row
     dev_args = [x.to(dev) for x in (q, kp, vp, bt, kv, cu, off)]
     got = paged_attention(*dev_args[:5], cu_q=dev_args[5], q_pos_offsets=dev_args[6]).cpu()
     assert bool(got[69, 1].isnan().all()) and bool(got[:, 2].isnan().all())
