@@ -81,7 +81,7 @@ __global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfm
     const uint16_t* __restrict__ kpool, const uint16_t* __restrict__ vpool,
     const int32_t* __restrict__ bt, int64_t bt_stride, const int32_t* __restrict__ kv_lens,
     const int32_t* __restrict__ cu_q, const int32_t* __restrict__ offsets, int B, int Hkv,
-    int64_t num_pages, float scale_log2) {
+    int64_t num_pages, float scale_log2, int maybe_alike) {
   constexpr int D = PF_D, P = PF_P, TILE = D * P;
   constexpr int NT = 64 * NW * KS;        // threads per workgroup
   constexpr int PPT = PF_WROWS * NW / G;  // query positions per work item
@@ -116,9 +116,37 @@ __global__ __launch_bounds__(64 * NW * KS, 8 / (NW * KS)) void paged_prefill_mfm
     for (int x = 0; x < NW * KS; ++x) carry += wsum[x];
     __syncthreads();
   }
+  // where XCDs share heads and may deal out whole sequences: whether none has a quarter more work
+  // (rows times keys) than another
+  bool alike = false;
+  if (maybe_alike) {
+    __shared__ float wmin[NW * KS], wmax[NW * KS];
+    float least = INFINITY, most = 0.f;
+    for (int i = threadIdx.x; i < B; i += NT) {
+      const int n = cu_q ? cu_q[i + 1] - cu_q[i] : 1, L = kv_lens[i];
+      const float keys = offsets ? fmaxf(float(min(L, offsets[i] + n)) - 0.5f * n, 0.f) : float(L);
+      const float work = float(max(n, 0)) * (keys + PF_KT);
+      least = fminf(least, work);
+      most = fmaxf(most, work);
+    }
+    least = -wave_max(-least);
+    most = wave_max(most);
+    if (lane == 0) {
+      wmin[threadIdx.x >> 6] = least;
+      wmax[threadIdx.x >> 6] = most;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < NW * KS; ++x) {
+      least = fminf(least, wmin[x]);
+      most = fmaxf(most, wmax[x]);
+    }
+    // scalar: a per-lane item made every address of the kernel one
+    alike = __builtin_amdgcn_readfirstlane(most <= 1.25f * least ? 1 : 0) != 0;
+  }
   // this workgroup's item: its kv head, and item j of that head over the sequences in order
   int h, j;
-  if (!xcd_item(blockIdx.x, carry, Hkv, h, j)) return;
+  if (!xcd_item(blockIdx.x, carry, Hkv, h, j, alike)) return;
   int lo = 0, hi = B - 1;  // the sequence holding the item: the last with tile_pref[b] <= j
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -524,6 +552,10 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
   const bool split =
       !wide && bt_stride * PF_P >= PF_SPLIT_TABLE &&
       (ceil_div(total_q_rows, 4 * PF_WROWS / G) + num_seqs) * Hkv <= device_cus();
+  // equal chunks of as many sequences as XCDs share a head, or a multiple (the kernel looks at their
+  // keys; unequal ones rarely have such a sum, and are spared the look: 2-3 % of 50-100 us)
+  const int sharing = 8 / (Hkv % 8 == 0 ? 8 : Hkv % 4 == 0 ? 4 : Hkv % 2 == 0 ? 2 : 1);
+  const int maybe_alike = sharing > 1 && num_seqs % sharing == 0 && total_q_rows % num_seqs == 0;
   // work items: at most ceil(total rows / ppt) + one partial item per sequence
   const int64_t items = (ceil_div(total_q_rows, ppt) + num_seqs) * Hkv;
   const int64_t blocks = ceil_div(items, 8) * 8;
@@ -535,7 +567,7 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
                      reinterpret_cast<uint16_t*>(out), reinterpret_cast<const uint16_t*>(q),   \
                      reinterpret_cast<const uint16_t*>(k_pages),                               \
                      reinterpret_cast<const uint16_t*>(v_pages), bt, bt_stride, kv_lens, cu_q, \
-                     offsets, num_seqs, Hkv, num_pages, scale_log2)
+                     offsets, num_seqs, Hkv, num_pages, scale_log2, maybe_alike)
 #define PIA_PF_G(NW, KS)                  \
   switch (G) {                            \
     case 1: PIA_PF(1, NW, KS); break;     \

@@ -134,3 +134,23 @@ def test_table_width_changes_nothing(dev, rows, ctx):
     wide[:, :bt.shape[1]] = bt
     assert torch.equal(paged_attention(q, kp, vp, bt, kv, cu_q=cu, q_pos_offsets=off),
                        paged_attention(q, kp, vp, wide, kv, cu_q=cu, q_pos_offsets=off))
+
+
+@pytest.mark.parametrize("rows,ctx,Hq,Hkv,dtype", [
+    # kv heads that XCDs share (4, 10, 6, 3 heads: two, four, four, eight XCDs a head): sequences alike,
+    # dealt out in runs; of equal rows but other contexts, and of other rows, item by item
+    ([70] * 4, [30] * 4, 32, 4, torch.bfloat16),
+    ([130] * 2, [300, 290], 16, 4, torch.float16),
+    ([65] * 8, [0] * 8, 20, 10, torch.bfloat16),
+    ([33] * 4, [100] * 4, 48, 6, torch.bfloat16),
+    ([40] * 8, [16] * 8, 12, 3, torch.float16),
+    ([70] * 4, [0, 600, 10, 300], 32, 4, torch.bfloat16),
+    ([1, 139, 70, 70], [0, 0, 64, 1], 20, 10, torch.bfloat16),
+    ([50] * 3, [20] * 3, 12, 3, torch.bfloat16),
+])
+def test_work_lists(dev, rows, ctx, Hq, Hkv, dtype):
+    args = _case(dev, rows, ctx, Hq, Hkv, dtype, 9)
+    q, kp, vp, bt, kv, cu, off = (x.to(dev) for x in args)
+    got = paged_attention(q, kp, vp, bt, kv, cu_q=cu, q_pos_offsets=off).double().cpu()
+    tol = 2.0 * args[2].abs().max().item() * (2 ** -8 if dtype == torch.bfloat16 else 2 ** -11)
+    assert (got - _ref(*args)).abs().max().item() <= tol
