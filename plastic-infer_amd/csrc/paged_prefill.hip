@@ -533,13 +533,23 @@ int launch_prefill_mfma(int dtype, void* out, const void* q, const void* k_pages
                         int64_t total_q_rows, int Hq, int Hkv, int64_t num_pages,
                         float scale_log2, hipStream_t s) {
   const int G = Hq / Hkv;
-  // eight waves (256 rows per item, one K / V tile staged for all of them) when the sequences
-  // average at least half an item and the items fill the compute units twice over, else four
-  // (128 rows): 312 items of 8 sequences of 100..800 rows, 16/8 heads, 75.8 us against 64.9 with
-  // four; 72 items of one sequence of 300 rows behind 1500 tokens, 32/8 heads, 63.5 against 55.2
+  // Eight waves (256 rows per item, one K / V tile staged for all of them) or four (128 rows), where
+  // the sequences average at least half of the larger item: two small items side by side take a
+  // compute unit a tenth longer than a large one, but leave fewer units idle and, of different
+  // lengths, pair long with short. So the large ones are for calls whose items fill the units
+  //  - twice (below that, 8 sequences of 100..800 rows, 16/8 heads, 312 items: 75.8 us, four waves
+  //    64.9; 72 items of one of 300 rows behind 1500 tokens, 32/8: 63.5 and 55.2), or
+  //  - once, whole and alike: chunks of equal whole items (two of 1024 rows behind 8192, 32/8 heads,
+  //    256 items: 280 us, four waves 322) or one with more before it than in it (1024 rows behind 4096,
+  //    64/8 heads: 157 and 171; without, all lengths: 37.3 with four waves, 40.1). Unequal ones: 4 of
+  //    254..766 rows, 32/8, 248 items: 33.2, four waves 32.2; 8 of 140..784, 16/8, 288: 61.2, 56.6.
   const int wide_ppt = 8 * PF_WROWS / G;
+  const int64_t cus = device_cus(), filled = ceil_div(total_q_rows, wide_ppt) * Hkv;
+  const bool even = num_seqs == 1 ? bt_stride * PF_P >= 2 * total_q_rows
+                                  : total_q_rows % (int64_t(wide_ppt) * num_seqs) == 0;
   const bool wide = 2 * total_q_rows >= int64_t(wide_ppt) * num_seqs &&
-                    (ceil_div(total_q_rows, wide_ppt) + num_seqs) * Hkv >= 2 * int64_t(device_cus());
+                    (filled + int64_t(num_seqs) * Hkv >= 2 * cus ||
+                     (even && filled <= cus && filled >= cus * 15 / 16));
   const int ppt = (wide ? 8 : 4) * PF_WROWS / G;
   // With no more items of four waves than compute units, two groups of waves share an item's keys:
   // its chain of tiles, which is the call's time then, is half as long, for a longer start and a

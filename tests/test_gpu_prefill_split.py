@@ -147,6 +147,9 @@ def test_table_width_changes_nothing(dev, rows, ctx):
     ([70] * 4, [0, 600, 10, 300], 32, 4, torch.bfloat16),
     ([1, 139, 70, 70], [0, 0, 64, 1], 20, 10, torch.bfloat16),
     ([50] * 3, [20] * 3, 12, 3, torch.bfloat16),
+    # equal chunks whose 256-row items fill the compute units once (a line in the launch)
+    ([512] * 4, [0] * 4, 32, 8, torch.bfloat16),
+    ([1024], [1200], 64, 8, torch.bfloat16),
 ])
 def test_work_lists(dev, rows, ctx, Hq, Hkv, dtype):
     args = _case(dev, rows, ctx, Hq, Hkv, dtype, 9)
