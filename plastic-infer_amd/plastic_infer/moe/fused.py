@@ -139,9 +139,9 @@ def _ffn(hidden_states, w1, w2, topk_weights, topk_ids, activation, on_input, ou
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     N.call("pia_moe_ffn_bank", N.ptr(out), N.ptr(route_out), hidden_states.data_ptr(),
            hidden_states.stride(0), w1.data_ptr(), w2.data_ptr(), weights.data_ptr(),
-           ids.data_ptr(), M, k, E, layer_experts or 0, H, inter, act, 1 if on_input else 0, dt, N.ptr(act_buffer),
-           0 if act_buffer is None else act_buffer.stride(0), ws.data_ptr(), ws_bytes,
-           N.stream_of(dev))
+           ids.data_ptr(), M, k, E, layer_experts or 0, H, inter, act, 1 if on_input else 0, dt,
+           N.ptr(act_buffer), 0 if act_buffer is None else act_buffer.stride(0), ws.data_ptr(),
+           ws_bytes, N.stream_of(dev))
 
 
 def _routed_ffn(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
